@@ -17,11 +17,9 @@
 // non-temporal streams: a hot expert's 128-row tasks run side by side and
 // share its weights through L2.
 //
-// GEMMs: the slab kernels' decomposition (gate/up: a workgroup of 8 waves
-// covers 8 gate/up tile pairs of one task; down: 16-channel output tiles)
-// with up to 8 MFMA row tiles per weight fragment.  The gate/up chain costs
-// a v_cvt and a v_fma per accumulator element and group, so at 128 rows the
-// kernel is VALU-bound (~1/4 of int8 MFMA peak); down W8 is MFMA/HBM-bound.
+// GEMMs: W4 in groups of 32 runs the int8 contract on fp16 MFMA, every other
+// grouped format on 32x32 int8 MFMA, W8 per-channel down on 16x16 int8 MFMA,
+// all with up to 128 rows of a task per weight fragment.
 #include "q38m_device.h"
 #include "q38m_internal.h"
 #include "q38m_select.h"
@@ -292,276 +290,37 @@ __global__ __launch_bounds__(64) void wide_scatter_kernel(const int32_t* __restr
 
 // ---- workgroup placement -----------------------------------------------------
 
-// The grouped GEMMs below run on (slice, task) grids: gridDim.x slices of
-// the output channels times one row per task slot.  The dispatcher hands
-// workgroups to the 8 XCDs round-robin by linear id, and each XCD has its
-// own L2.  This maps the live pairs (task < the plan's task count) so that
-// each XCD runs one contiguous range of them: a task's slices read the same
-// rows, and an expert's consecutive tasks read the same weights, from one
-// L2.  Workgroups past the live pairs return at once, spread evenly over
-// the XCDs.
+// The grouped GEMMs below run on one-dimensional grids of (task, slice)
+// pairs, `slices` slices of the output channels per task slot.  The
+// dispatcher hands workgroups to the 8 XCDs round-robin by id, and each XCD
+// has its own L2: XCD x gets the blocks of kTaskBlock consecutive tasks x,
+// x + 8, x + 16, ..., a task's slices next to each other, so that the slices
+// read the same rows, and an expert's neighbouring tasks the same weights,
+// from one L2.  Small blocks keep the XCDs' loads alike (contiguous eighths
+// of the tasks differ by 10-30 % in rows for 1,500 to 6,000 tokens), and the
+// map needs no word of the plan, so a workgroup's first read is its task
+// record; slots past the plan's tasks hold zero records.
 struct Placement {
     uint32_t task, slice;
 };
 
-__device__ inline bool place_on_xcds(const uint32_t* live_tasks, Placement& at) {
-    constexpr uint32_t kXcds = 8;
-    const uint32_t slices = gridDim.x;
-    const uint32_t live = min(*live_tasks, gridDim.y) * slices;
-    const uint32_t id = blockIdx.y * slices + blockIdx.x;
-    if (id >= live) return false;
-    const uint32_t per = live / kXcds, extra = live % kXcds;
-    const uint32_t xcd = id % kXcds;
-    const uint32_t j = xcd * per + min(xcd, extra) + id / kXcds;
-    at.task = j / slices;
-    at.slice = j % slices;
-    return true;
+constexpr uint32_t kXcds = 8;
+constexpr uint32_t kTaskBlock = 4;
+
+__host__ __device__ constexpr uint32_t placed_workgroups(uint32_t task_slots, uint32_t slices) {
+    constexpr uint32_t kRound = kXcds * kTaskBlock;
+    return (task_slots + kRound - 1u) / kRound * kRound * slices;
+}
+
+__device__ inline bool place_on_xcds(uint32_t task_slots, uint32_t slices, Placement& at) {
+    const uint32_t xcd = blockIdx.x % kXcds, j = blockIdx.x / kXcds;
+    const uint32_t within = j % (kTaskBlock * slices);
+    at.task = (j / (kTaskBlock * slices) * kXcds + xcd) * kTaskBlock + within / slices;
+    at.slice = within % slices;
+    return at.task < task_slots;
 }
 
 // ---- gate/up ----------------------------------------------------------------
-
-struct TileQuad {
-    uint4 w;  // one 16-channel tile's data of one quad
-    uint2 s;  // its scale words (4, 2 or 1 groups; load_quad_scales)
-};
-
-// Gate/up, W4, over a task of up to 128 rows.  A workgroup of 16 waves
-// covers 8 gate/up channel pairs (16 channels each) of one task; wave w
-// owns pair w % 8 for rows 64 (w / 8) .. +63 (up to 4 row tiles of 16) and
-// runs both the pair's gate tile and its up tile, so each A fragment feeds
-// two MFMAs and the SwiGLU epilogue stays in registers.
-//
-// Per quad (128 columns of K) the workgroup stages into LDS the task's 128
-// int8 rows (16 KB), its 16 weight tiles (16 KB) and their scale words;
-// every thread moves one 16-byte row piece, one 16-byte weight piece and
-// one 4-byte scale piece.  Those loads are issued two quads ahead into two
-// register sets and stored one quad ahead into a double-buffered image, and
-// the barrier between quads waits only for LDS operations, so the global
-// loads of later quads stay in flight across it (a full workgroup fence
-// would wait for them).
-//
-// Arithmetic per scale group and tile: kSub v_mfma_i32_16x16x32_i8 chained
-// through the accumulator, started from the bits of 1.5 * 2^23 so that the
-// result read as a float is 12582912 + acc exactly (|acc| < 2^22); one
-// v_add_f32 recovers (float)acc and one v_fma_f32 continues the group chain
-// -- the contract's y = fmaf((float)acc_g, s_g, y) in group order.  The
-// next tile's MFMAs are issued before this tile's fp32 step.  The W4
-// nibbles sit in the high half of each int8 (16 * w); fp16 scales run the
-// chain on 16 * y, bf16 scales take s / 16.  Per-row token scale and route
-// weight are staged in LDS once for the epilogue.
-template <uint32_t H, uint32_t I, uint32_t kSub, bool kBf16>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4)))
-void gate_up_w4_wide_kernel(const uint4* __restrict__ w, const uint16_t* __restrict__ s,
-                            const int8_t* __restrict__ xq, const float* __restrict__ xs,
-                            const uint32_t* __restrict__ packed,
-                            const float* __restrict__ route_weights,
-                            const q38m_task_v1* __restrict__ tasks, const uint32_t* __restrict__ live_tasks, uint16_t* __restrict__ mid) {
-    constexpr uint32_t kQuads = H / 128u;
-    constexpr uint32_t kTilesAll = 2u * I / 16u;
-    constexpr uint32_t kRowScales = 4u / kSub;                           // words per row per quad
-    constexpr uint32_t kGroups = 4u / kSub;                              // scale groups per quad
-    constexpr uint32_t kScalePieces = 16u * 16u * kRowScales * 2u / 4u;  // 4-byte pieces per quad
-    static_assert(kQuads % 2u == 0u, "two staging register sets");
-    static_assert(kScalePieces <= 1024u, "one scale piece per thread");
-    // per buffer: A [sub-block j][row tile][lane] 8-byte MFMA fragments, the
-    // workgroup's 16 weight tiles [tile][lane] and their scale words
-    __shared__ __align__(16) uint2 a_lds[2][4u * kRowTiles * 64u];
-    __shared__ __align__(16) uint4 w_lds[2][16u * 64u];
-    __shared__ __align__(16) uint32_t s_lds[2][kScalePieces];
-    __shared__ float2 row_info[kWideRows];  // (token scale, route weight)
-
-    Placement at;
-    if (!place_on_xcds(live_tasks, at)) return;
-    const TaskRecord task = read_task(tasks, at.task);
-    const uint32_t rows = task.rows;
-    if (rows == 0u) return;
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t rh = wave >> 3;
-    const uint32_t pr = wave & 7u;
-    const uint32_t n = lane & 15u, qh = lane >> 4;
-    const uint32_t e = task.expert;
-    const uint32_t p0 = task.begin;
-    const int here = static_cast<int>(rows) - static_cast<int>(64u * rh);
-    const uint32_t nt = __builtin_amdgcn_readfirstlane(
-        here <= 0 ? 0u : (here >= 64 ? 4u : (static_cast<uint32_t>(here) + 15u) / 16u));
-
-    // staging: row piece (row tid/8, 16-byte chunk tid%8), weight piece
-    // (slot tid/64 of the workgroup's 16, lane tid%64), scale piece tid
-    const uint32_t sr = tid >> 3, sch = tid & 7u;
-    const bool alive = sr < rows;
-    const uint32_t assignment = alive ? checked(packed[p0 + sr], Q38M_WIDE_MAX_TOKENS * kTopK, kCheckToken) : 0u;
-    if (sch == 0u && alive)
-        row_info[sr] = make_float2(xs[assignment / kTopK], route_weights[assignment]);
-    const uint4* a_src =
-        reinterpret_cast<const uint4*>(xq + static_cast<size_t>(assignment / kTopK) * H) + sch;
-    const uint32_t a_at = ((sch >> 1) * kRowTiles + (sr >> 4)) * 64u + (sch & 1u) * 32u + (sr & 15u);
-    const size_t slot0 = static_cast<size_t>(e) * kQuads * kTilesAll + at.slice * 16u;
-    const uint4* w_src = w + slot0 * 64u + tid;
-    const uint32_t* s_src = reinterpret_cast<const uint32_t*>(s) + slot0 * 16u * kRowScales / 2u + tid;
-    const bool s_thread = tid < kScalePieces;
-    struct Stage {
-        uint4 a, w;
-        uint32_t s;
-    };
-    auto load_stage = [&](uint32_t kq) __attribute__((always_inline)) {
-        Stage st;
-        st.a = alive ? a_src[kq * 8u] : make_uint4(0u, 0u, 0u, 0u);
-        st.w = w_src[static_cast<size_t>(kq) * kTilesAll * 64u];
-        st.s = s_thread ? s_src[static_cast<size_t>(kq) * kTilesAll * 16u * kRowScales / 2u] : 0u;
-        return st;
-    };
-    auto store_stage = [&](const Stage& st, uint32_t buffer) __attribute__((always_inline)) {
-        a_lds[buffer][a_at] = make_uint2(st.a.x, st.a.y);
-        a_lds[buffer][a_at + 16u] = make_uint2(st.a.z, st.a.w);
-        w_lds[buffer][tid] = st.w;
-        if (s_thread) s_lds[buffer][tid] = st.s;
-    };
-
-    float y[4][2][4];
-#pragma unroll
-    for (uint32_t t = 0; t < 4u; ++t)
-#pragma unroll
-        for (uint32_t u = 0; u < 2u; ++u)
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i) y[t][u][i] = 0.0f;
-    v4i bias;
-    bias.x = bias.y = bias.z = bias.w = 0x4B400000;
-    float unbias;  // -12582912.0f in a scalar register (no literal per use)
-    asm volatile("s_mov_b32 %0, 0xcb400000" : "=s"(unbias));
-
-    // One quad for kNt row tiles.  Chain k = (scale group gg, row tile t,
-    // gate/up u); the A fragments of (gg, t) are read one set ahead and a
-    // group's B fragments are unpacked once for all row tiles.
-    auto multiply = [&](auto tiles, uint32_t buffer) __attribute__((always_inline)) {
-        constexpr uint32_t kNt = decltype(tiles)::value;
-        constexpr uint32_t kSets = kGroups * kNt;
-        constexpr uint32_t kChains = kSets * 2u;
-        const uint2* abuf = a_lds[buffer] + lane;
-        const uint4 gq = w_lds[buffer][(2u * pr) * 64u + lane];
-        const uint4 uq = w_lds[buffer][(2u * pr + 1u) * 64u + lane];
-        const uint16_t* sbase = reinterpret_cast<const uint16_t*>(s_lds[buffer]);
-        const uint2 gs = load_quad_scales<kSub, false>(sbase + ((2u * pr) * 16u + n) * kRowScales);
-        const uint2 us =
-            load_quad_scales<kSub, false>(sbase + ((2u * pr + 1u) * 16u + n) * kRowScales);
-        const uint32_t gw[4] = {gq.x, gq.y, gq.z, gq.w};
-        const uint32_t uw[4] = {uq.x, uq.y, uq.z, uq.w};
-        float sc[2][kGroups];
-#pragma unroll
-        for (uint32_t gg = 0; gg < kGroups; ++gg) {
-#pragma unroll
-            for (uint32_t u = 0; u < 2u; ++u) {
-                const uint32_t word = quad_scale_word(u ? us : gs, gg);
-                sc[u][gg] = kBf16 ? bf16_to_f32(word) * 0.0625f : f16_to_f32(word);
-                asm volatile("" : "+v"(sc[u][gg]));  // a plain v_fma_f32, not v_fma_mix
-            }
-        }
-        long fa[2][kSub];
-        auto read_set = [&](uint32_t m) __attribute__((always_inline)) {
-            const uint32_t gg = m / kNt, t = m % kNt;
-#pragma unroll
-            for (uint32_t sb = 0; sb < kSub; ++sb)
-                fa[m & 1u][sb] = as_long(abuf[((gg * kSub + sb) * kRowTiles + 4u * rh + t) * 64u]);
-        };
-        long bf[2][kSub];
-        v4i d[2];
-        auto issue = [&](uint32_t k) __attribute__((always_inline)) {
-            const uint32_t m = k / 2u, u = k & 1u;
-            const uint32_t gg = m / kNt, t = m % kNt;
-            if (u == 0u) {
-                if (m + 1u < kSets) read_set(m + 1u);
-                if (t == 0u) {
-#pragma unroll
-                    for (uint32_t sb = 0; sb < kSub; ++sb) {
-                        bf[0][sb] = unpack_w4x16(gw[gg * kSub + sb]);
-                        bf[1][sb] = unpack_w4x16(uw[gg * kSub + sb]);
-                    }
-                }
-            }
-            v4i acc = bias;
-#pragma unroll
-            for (uint32_t sb = 0; sb < kSub; ++sb)
-                acc = mfma_i8_16x16x32(fa[m & 1u][sb], bf[u][sb], acc);
-            d[k & 1u] = acc;
-        };
-        auto step = [&](uint32_t k) __attribute__((always_inline)) {
-            const uint32_t m = k / 2u, u = k & 1u;
-            const uint32_t gg = m / kNt, t = m % kNt;
-            const float scale = sc[u][gg];
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i)
-                y[t][u][i] =
-                    __builtin_fmaf(__int_as_float(d[k & 1u][i]) + unbias, scale, y[t][u][i]);
-            // keep the chain step here, between this tile's MFMAs and the next
-            // ones (otherwise it can sink to the end of the loop body, and
-            // every accumulator of the quad stays live until then)
-            asm volatile("" : "+v"(y[t][u][0]), "+v"(y[t][u][1]), "+v"(y[t][u][2]),
-                         "+v"(y[t][u][3]));
-        };
-        read_set(0);
-#pragma unroll
-        for (uint32_t k = 0; k <= kChains; ++k) {
-            if (k < kChains) issue(k);
-            __builtin_amdgcn_sched_barrier(0);
-            if (k > 0u) step(k - 1u);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    // barrier over LDS only: this wave's LDS operations are complete, its
-    // global loads (the staging of later quads) stay in flight
-    auto lds_barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-
-    // quad q: loaded at the start of quad q-2 into register set q%2, stored
-    // at the end of quad q-1 into LDS buffer q%2, multiplied during quad q.
-    // The loop is instantiated per row-tile count (three tiles run as four,
-    // one as two; the extra rows are zero), so a wave's accumulators keep
-    // one register assignment through it; every instance passes the same
-    // barriers.
-    Stage set0 = load_stage(0), set1 = load_stage(1);
-    store_stage(set0, 0u);
-    __syncthreads();
-    auto k_loop = [&](auto tiles) __attribute__((always_inline)) {
-        constexpr uint32_t kNt = decltype(tiles)::value;
-#pragma unroll 1
-        for (uint32_t kq = 0; kq < kQuads; kq += 2u) {
-            if (kq + 2u < kQuads) set0 = load_stage(kq + 2u);
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (kNt > 0u) multiply(tiles, 0u);
-            store_stage(set1, 1u);
-            lds_barrier();
-            if (kq + 3u < kQuads) set1 = load_stage(kq + 3u);
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (kNt > 0u) multiply(tiles, 1u);
-            if (kq + 2u < kQuads) store_stage(set0, 0u);
-            lds_barrier();
-        }
-    };
-    if (nt > 2u)
-        k_loop(std::integral_constant<uint32_t, 4>{});
-    else if (nt > 0u)
-        k_loop(std::integral_constant<uint32_t, 2>{});
-    else
-        k_loop(std::integral_constant<uint32_t, 0>{});
-
-    // SwiGLU: D lane (qh, n) holds rows 4qh + i of each tile, channel n
-    const uint32_t channel = (at.slice * 8u + pr) * 16u + n;
-    const float unscale = kBf16 ? 1.0f : 0.0625f;
-#pragma unroll
-    for (uint32_t t = 0; t < 4u; ++t) {
-        if (t >= nt) break;
-#pragma unroll
-        for (uint32_t i = 0; i < 4u; ++i) {
-            const uint32_t r = 64u * rh + 16u * t + 4u * qh + i;
-            if (r >= rows) continue;
-            const float2 info = row_info[r];
-            const float yg = (y[t][0][i] * unscale) * info.x;
-            const float yu = (y[t][1][i] * unscale) * info.x;
-            mid[static_cast<size_t>(p0 + r) * I + channel] =
-                static_cast<uint16_t>(swiglu_fold(yg, yu, info.y));
-        }
-    }
-}
 
 // ---- gate/up, W4 groups of 32, on fp16 MFMA --------------------------------
 //
@@ -569,7 +328,7 @@ void gate_up_w4_wide_kernel(const uint4* __restrict__ w, const uint16_t* __restr
 // as 16 * w in [-128, 112]) are exact in fp16, their products (< 2^14) and
 // every partial sum of a 32-wide group (< 2^19) exact in fp32, so
 // v_mfma_f32_16x16x32_f16 returns (float)(16 * acc_g) itself -- the value
-// the int8 MFMA path recovers with one extra VALU op per accumulator element
+// an int8 MFMA path recovers with one extra VALU op per accumulator element
 // and group.  The chain step is then a single v_fma_f32, and the MFMA runs
 // at the same 16 cycles as v_mfma_i32_16x16x32_i8.
 //
@@ -666,8 +425,7 @@ __device__ __forceinline__ v4f mfma_f16_16x16x32(uint4 a, uint4 b, v4f c) {
 // The barrier between steps waits for LDS operations only.  Two workgroups
 // share a CU (8 waves each at 4 waves per SIMD), so one's barriers,
 // prologue and epilogue overlap the other's MFMAs.  fp16 scales carry
-// 16 * y, bf16 scales take s / 16, as in the int8 kernel above; the
-// epilogue is the same.
+// 16 * y (exact: far from the subnormal range), bf16 scales take s / 16.
 template <uint32_t H, uint32_t I, bool kBf16>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
 void gate_up_w4g32_f16_kernel(const uint4* __restrict__ w, const uint16_t* __restrict__ s,
@@ -675,7 +433,7 @@ void gate_up_w4g32_f16_kernel(const uint4* __restrict__ w, const uint16_t* __res
                               const uint32_t* __restrict__ packed,
                               const float* __restrict__ route_weights,
                               const q38m_task_v1* __restrict__ tasks,
-                              const uint32_t* __restrict__ live_tasks, uint16_t* __restrict__ mid) {
+                              uint32_t task_slots, uint16_t* __restrict__ mid) {
     constexpr uint32_t kHalves = H / 64u;  // staging steps
     constexpr uint32_t kTilesAll = 2u * I / 16u;
     constexpr uint32_t kWgTiles = 16u;  // 8 pairs
@@ -689,7 +447,7 @@ void gate_up_w4g32_f16_kernel(const uint4* __restrict__ w, const uint16_t* __res
     __shared__ float2 row_info[kWideRows];  // (token scale, route weight)
 
     Placement at;
-    if (!place_on_xcds(live_tasks, at)) return;
+    if (!place_on_xcds(task_slots, I / 16u / 8u, at)) return;
     const TaskRecord task = read_task(tasks, at.task);
     const uint32_t rows = task.rows;
     if (rows == 0u) return;
@@ -890,225 +648,6 @@ void gate_up_w4g32_f16_kernel(const uint4* __restrict__ w, const uint16_t* __res
     }
 }
 
-// Gate/up, W8 (paired K-block-major layout; the reference's edge-layer
-// format) over a task of up to 128 rows: the W4 kernel's plan with 64-wide
-// K blocks -- 16 waves (8 gate tiles, 8 up tiles), one tile per wave for
-// kTiles 16-row tiles, A staged one K block (8 KiB) at a time into a
-// double-buffered LDS image [row tile][lane] of 16-byte fragments, weights
-// two blocks ahead.  Groups of one block (64 columns): per tile one
-// v_mfma_i32_16x16x64_i8 from zero, then y = fma((float)acc, s_g, y) with
-// the MFMA/fma interleave pinned; groups of two blocks or per channel: each
-// tile's int32 accumulator chains through the MFMA input (kTiles more
-// registers) and joins the chain at the group's last block (per channel:
-// y = (float)acc * s at the end).  Scales in the artifact order.
-template <uint32_t H, uint32_t I, uint32_t kThreads, uint32_t kTiles, uint32_t kBlocksPerGroup,
-          bool kBf16>
-__device__ __forceinline__ void gate_up_w8_wide_rows(
-    const uint4* __restrict__ wbase, const uint16_t* __restrict__ srow,
-    const int8_t* __restrict__ xq, const float* __restrict__ xs,
-    const uint32_t* __restrict__ packed, const float* __restrict__ route_weights,
-    uint16_t* __restrict__ mid, uint4 (*a_lds)[kRowTiles * 64u], float* gate_lds,
-    uint32_t rows, uint32_t p0, uint32_t pair, bool up) {
-    constexpr uint32_t kBlocks = H / 64u;
-    constexpr uint32_t kBlockWords = 2u * I / 16u * 64u;  // uint4 per K block of one expert
-    constexpr bool kPerChannel = kBlocksPerGroup == kBlocks;
-    constexpr uint32_t kPieces = kTiles * 16u * 4u;  // 16-byte row pieces per block
-    constexpr uint32_t kPerThread = (kPieces + kThreads - 1u) / kThreads;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t n = lane & 15u;
-    const uint32_t q = lane >> 4;
-    const uint32_t wave_in_half = (threadIdx.x >> 6) & 7u;
-    const v4i zero = {0, 0, 0, 0};
-
-    struct Block {
-        uint4 w;     // the tile's 16 bytes of one K block
-        uint32_t s;  // the scale word of the block's group
-    };
-    auto load = [&](uint32_t kb) {
-        const uint32_t k = kb < kBlocks ? kb : kBlocks - 1u;  // past the end: re-read (L1 hit)
-        const uint32_t g = kPerChannel ? 0u : k / kBlocksPerGroup;
-        return Block{wbase[k * kBlockWords + lane], static_cast<uint32_t>(srow[g])};
-    };
-
-    // Piece i: row r = i/4, 16-byte piece c = i%4 of the row's 64 bytes of
-    // the block (lane group c).  Rows past valid_rows stage zeros.
-    const uint4* row_src[kPerThread];
-    uint32_t lds_at[kPerThread];
-    bool alive[kPerThread], staged[kPerThread];
-#pragma unroll
-    for (uint32_t u = 0; u < kPerThread; ++u) {
-        const uint32_t i = threadIdx.x + u * kThreads;
-        const uint32_t r = i / 4u, c = i % 4u;
-        staged[u] = i < kPieces;
-        alive[u] = staged[u] && r < rows;
-        const uint32_t token = alive[u] ? checked(packed[p0 + r], Q38M_WIDE_MAX_TOKENS * kTopK, kCheckToken) / kTopK : 0u;
-        row_src[u] = reinterpret_cast<const uint4*>(xq + static_cast<size_t>(token) * H) + c;
-        lds_at[u] = (r / 16u) * 64u + c * 16u + r % 16u;
-    }
-    uint4 pieces[kPerThread];
-    auto load_a = [&](uint32_t kb) {
-#pragma unroll
-        for (uint32_t u = 0; u < kPerThread; ++u)
-            pieces[u] = alive[u] ? row_src[u][kb * 4u] : make_uint4(0u, 0u, 0u, 0u);
-    };
-    auto store_a = [&](uint32_t buffer) {
-#pragma unroll
-        for (uint32_t u = 0; u < kPerThread; ++u)
-            if (staged[u]) a_lds[buffer][lds_at[u]] = pieces[u];
-    };
-
-    float y[kTiles][4];
-    v4i acc[kTiles];  // groups of two blocks / per channel: the running int32 tiles
-#pragma unroll
-    for (uint32_t t = 0; t < kTiles; ++t) {
-        acc[t] = zero;
-#pragma unroll
-        for (uint32_t i = 0; i < 4u; ++i) y[t][i] = 0.0f;
-    }
-
-    auto multiply = [&](uint32_t kb, const Block& b) {
-        const uint4* abuf = a_lds[kb & 1u] + lane;
-        const v4i bw = as_v4i(b.w);
-        const float scale = kBf16 ? bf16_to_f32(b.s) : f16_to_f32(b.s);
-        if constexpr (kBlocksPerGroup == 1u) {
-            v4i d[2];
-            d[0] = mfma_i8_16x16x64(as_v4i(abuf[0]), bw, zero);
-#pragma unroll
-            for (uint32_t t = 0; t < kTiles; ++t) {
-                if (t + 1u < kTiles)
-                    d[(t + 1u) & 1u] = mfma_i8_16x16x64(as_v4i(abuf[(t + 1u) * 64u]), bw, zero);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    y[t][i] = __builtin_fmaf(static_cast<float>(d[t & 1u][i]), scale, y[t][i]);
-                asm volatile("" : "+v"(y[t][0]), "+v"(y[t][1]), "+v"(y[t][2]), "+v"(y[t][3]));
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        } else {
-            const bool first = kb % kBlocksPerGroup == 0u;
-#pragma unroll
-            for (uint32_t t = 0; t < kTiles; ++t)
-                acc[t] = mfma_i8_16x16x64(as_v4i(abuf[t * 64u]), bw, first ? zero : acc[t]);
-            if constexpr (!kPerChannel) {
-                if (kb % kBlocksPerGroup == kBlocksPerGroup - 1u) {
-#pragma unroll
-                    for (uint32_t t = 0; t < kTiles; ++t)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            y[t][i] = __builtin_fmaf(static_cast<float>(acc[t][i]), scale, y[t][i]);
-                }
-            }
-        }
-    };
-    // one block: weights two ahead into the set just consumed, A one ahead
-    auto step = [&](uint32_t kb, const Block& cur, Block& refill) {
-        refill = load(kb + 2u);
-        if (kb + 1u < kBlocks) load_a(kb + 1u);
-        __builtin_amdgcn_sched_barrier(0);
-        multiply(kb, cur);
-        if (kb + 1u < kBlocks) store_a((kb + 1u) & 1u);
-        __syncthreads();
-    };
-
-    load_a(0);
-    Block r0 = load(0), r1 = load(1), r2;
-    store_a(0);
-    __syncthreads();
-    static_assert(kBlocks % 3u == 2u, "three-set rotation plus two peeled blocks");
-#pragma unroll 1
-    for (uint32_t kb = 0; kb + 2u < kBlocks; kb += 3u) {
-        step(kb, r0, r2);
-        step(kb + 1u, r1, r0);
-        step(kb + 2u, r2, r1);
-    }
-    step(kBlocks - 2u, r0, r2);
-    multiply(kBlocks - 1u, r1);
-    if constexpr (kPerChannel) {
-        const float scale = kBf16 ? bf16_to_f32(r1.s) : f16_to_f32(r1.s);
-#pragma unroll
-        for (uint32_t t = 0; t < kTiles; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) y[t][i] = static_cast<float>(acc[t][i]) * scale;
-    }
-
-    // gate waves hand y over: gate_lds[pair in workgroup][row][channel],
-    // over the A image, once every wave has finished reading it
-    float* handoff = gate_lds + wave_in_half * (kWideRows * 16u);
-    __syncthreads();
-    if (!up) {
-#pragma unroll
-        for (uint32_t t = 0; t < kTiles; ++t)
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i) handoff[(16u * t + 4u * q + i) * 16u + n] = y[t][i];
-    }
-    __syncthreads();
-    if (!up) return;
-    const uint32_t channel = pair * 16u + n;
-#pragma unroll
-    for (uint32_t t = 0; t < kTiles; ++t) {
-#pragma unroll
-        for (uint32_t i = 0; i < 4u; ++i) {
-            const uint32_t r = 16u * t + 4u * q + i;
-            if (r >= rows) continue;
-            const uint32_t p = p0 + r;
-            const uint32_t a = checked(packed[p], Q38M_WIDE_MAX_TOKENS * kTopK, kCheckToken);
-            const float st = xs[a / kTopK];
-            mid[static_cast<size_t>(p) * I + channel] = static_cast<uint16_t>(
-                swiglu_fold(handoff[r * 16u + n] * st, y[t][i] * st, route_weights[a]));
-        }
-    }
-}
-
-template <uint32_t H, uint32_t I, uint32_t kPairs, uint32_t kBlocksPerGroup, bool kBf16>
-__global__ __launch_bounds__(kPairs * 128) __attribute__((amdgpu_waves_per_eu(4)))
-void gate_up_w8_wide_kernel(
-    const uint4* __restrict__ w, const uint16_t* __restrict__ s,
-    const int8_t* __restrict__ xq, const float* __restrict__ xs,
-    const uint32_t* __restrict__ packed, const float* __restrict__ route_weights,
-    const q38m_task_v1* __restrict__ tasks, const uint32_t* __restrict__ live_tasks, uint16_t* __restrict__ mid) {
-    constexpr uint32_t kBlocks = H / 64u;
-    constexpr uint32_t kSlots = 2u * I / 16u;
-    constexpr uint32_t kGroups = kBlocks / kBlocksPerGroup;
-    constexpr uint32_t kThreads = kPairs * 128u;
-    // the A image (two blocks) and, after the K loop, the gate hand-off
-    constexpr uint32_t kABytes = 2u * kRowTiles * 64u * 16u;
-    constexpr uint32_t kHandoffBytes = kPairs * kWideRows * 16u * 4u;
-    __shared__ __align__(16) uint8_t lds[kABytes > kHandoffBytes ? kABytes : kHandoffBytes];
-    auto a_lds = reinterpret_cast<uint4 (*)[kRowTiles * 64u]>(lds);
-    float* gate_lds = reinterpret_cast<float*>(lds);
-
-    Placement at;
-    if (!place_on_xcds(live_tasks, at)) return;
-    const TaskRecord task = read_task(tasks, at.task);
-    const uint32_t rows = task.rows;
-    if (rows == 0u) return;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const bool up = wave >= kPairs;
-    const uint32_t pair = at.slice * kPairs + (wave % kPairs);
-    const uint32_t e = task.expert;
-    const uint32_t p0 = task.begin;
-    const uint32_t n = threadIdx.x & 15u;
-    // paired K-block-major layout: for block kb the gate tile of pair p is
-    // slot 2p and its up tile slot 2p+1
-    const uint32_t slot = 2u * pair + (up ? 1u : 0u);
-    const uint4* wbase = w + (static_cast<size_t>(e) * kBlocks * kSlots + slot) * 64u;
-    const uint16_t* srow =
-        s + (static_cast<size_t>(e) * 2u * I + (up ? I : 0u) + pair * 16u + n) * kGroups;
-    const uint32_t tiles = (rows + 15u) / 16u;  // uniform per workgroup
-    auto run = [&](auto row_tiles) {
-        gate_up_w8_wide_rows<H, I, kThreads, decltype(row_tiles)::value, kBlocksPerGroup, kBf16>(
-            wbase, srow, xq, xs, packed, route_weights, mid, a_lds, gate_lds, rows, p0, pair, up);
-    };
-    if (tiles > 4u)
-        run(std::integral_constant<uint32_t, 8>{});
-    else if (tiles > 2u)
-        run(std::integral_constant<uint32_t, 4>{});
-    else if (tiles == 2u)
-        run(std::integral_constant<uint32_t, 2>{});
-    else
-        run(std::integral_constant<uint32_t, 1>{});
-}
-
 // ---- down -------------------------------------------------------------------
 
 // The route outputs of a chunk (fp32 [R][H], 2.68 GB for a config-5 layer)
@@ -1130,48 +669,23 @@ __device__ __forceinline__ void store_route_output(float* p, float v) {
 // ahead.  One A fragment is live at a time (row by row): holding all kRows
 // of them took the kernel to 256 VGPRs with spills (1.07 ms vs 1.00 ms on
 // a config-5 layer).  kRows (8, 4, 2 or 1 row tiles) is picked per task from its row
-// count.  Per channel (kBlocksPerGroup == I/64): o = ((float)acc * ws[e][c])
-// * sm[r], as the slab kernel.  Groups of 64 or 128 columns (kBlocksPerGroup
-// 1 or 2 K blocks): acc restarts at each group's first block and, at its
-// last, joins the fp32 chain y = fma((float)acc, s[e][c][g], y) in group
-// order; o = y * sm[r].
-template <uint32_t H, uint32_t I, uint32_t kTilesPerWave, uint32_t kRows,
-          uint32_t kBlocksPerGroup, bool kBf16>
+// count.  o = ((float)acc * ws[e][c]) * sm[r], as the slab kernel.
+template <uint32_t H, uint32_t I, uint32_t kTilesPerWave, uint32_t kRows, bool kBf16>
 __device__ __forceinline__ void down_w8_wide_rows(const uint4* __restrict__ wt,
                                                   const uint16_t* __restrict__ ws_expert,
                                                   const uint4* a_lds, const float* row_scale,
                                                   uint32_t rows, uint32_t p0, uint32_t tile0,
                                                   float* __restrict__ out) {
     constexpr uint32_t kBlocks = I / 64u;
-    constexpr bool kPerChannel = kBlocksPerGroup == kBlocks;
-    constexpr uint32_t kGroups = kBlocks / kBlocksPerGroup;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t n = lane & 15u;
     const uint32_t q = lane >> 4;
     const v4i zero = {0, 0, 0, 0};
-    // the tiles' scales of channel 16*(tile0+t)+n, artifact order
-    // [E][rows][groups]; per channel read after the K loop (fewer live VGPRs)
-    float ws[kTilesPerWave][kGroups];
-    auto load_scales = [&]() {
-#pragma unroll
-        for (uint32_t t = 0; t < kTilesPerWave; ++t)
-#pragma unroll
-            for (uint32_t g = 0; g < kGroups; ++g) {
-                const uint32_t word = ws_expert[((tile0 + t) * 16u + n) * kGroups + g];
-                ws[t][g] = kBf16 ? bf16_to_f32(word) : f16_to_f32(word);
-            }
-    };
-    if constexpr (!kPerChannel) load_scales();
     v4i acc[kTilesPerWave][kRows];
-    float y[kTilesPerWave][kRows][4];  // grouped: the fp32 chain
 #pragma unroll
     for (uint32_t t = 0; t < kTilesPerWave; ++t)
 #pragma unroll
-        for (uint32_t r = 0; r < kRows; ++r) {
-            acc[t][r] = zero;
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i) y[t][r][i] = 0.0f;
-        }
+        for (uint32_t r = 0; r < kRows; ++r) acc[t][r] = zero;
     // tile t's K block kb: wt[(t * kBlocks + kb) * 64]
     uint4 wq[3][kTilesPerWave];
     auto load_w = [&](uint32_t kb, uint4 (&dst)[kTilesPerWave]) {
@@ -1189,28 +703,17 @@ __device__ __forceinline__ void down_w8_wide_rows(const uint4* __restrict__ wt,
             const v4i a = as_v4i(a_lds[(kb * kRowTiles + r) * 64u + lane]);
 #pragma unroll
             for (uint32_t t = 0; t < kTilesPerWave; ++t)
-                acc[t][r] = mfma_i8_16x16x64(a, as_v4i(wq[kb % 3u][t]),
-                                             !kPerChannel && kb % kBlocksPerGroup == 0u
-                                                 ? zero
-                                                 : acc[t][r]);
-        }
-        if constexpr (!kPerChannel) {
-            if (kb % kBlocksPerGroup == kBlocksPerGroup - 1u) {
-#pragma unroll
-                for (uint32_t t = 0; t < kTilesPerWave; ++t)
-#pragma unroll
-                    for (uint32_t r = 0; r < kRows; ++r)
-#pragma unroll
-                        for (uint32_t i = 0; i < 4u; ++i)
-                            y[t][r][i] = __builtin_fmaf(static_cast<float>(acc[t][r][i]),
-                                                        ws[t][kb / kBlocksPerGroup], y[t][r][i]);
-            }
-            // one K block's tiles live at a time (unpinned, the zero-started
-            // blocks would all be issued at once)
-            __builtin_amdgcn_sched_barrier(0);
+                acc[t][r] = mfma_i8_16x16x64(a, as_v4i(wq[kb % 3u][t]), acc[t][r]);
         }
     }
-    if constexpr (kPerChannel) load_scales();
+    // the tiles' scales of channel 16*(tile0+t)+n, read after the K loop
+    // (fewer live VGPRs)
+    float ws[kTilesPerWave];
+#pragma unroll
+    for (uint32_t t = 0; t < kTilesPerWave; ++t) {
+        const uint32_t word = ws_expert[(tile0 + t) * 16u + n];
+        ws[t] = kBf16 ? bf16_to_f32(word) : f16_to_f32(word);
+    }
     // a row's kTilesPerWave adjacent 16-channel pieces go out in consecutive
     // stores, so its 64*kTilesPerWave bytes meet in L2 as whole lines
 #pragma unroll
@@ -1223,18 +726,15 @@ __device__ __forceinline__ void down_w8_wide_rows(const uint4* __restrict__ wt,
             float* dst = out + static_cast<size_t>(p0 + row) * H + tile0 * 16u + n;
 #pragma unroll
             for (uint32_t t = 0; t < kTilesPerWave; ++t)
-                store_route_output(dst + 16u * t,
-                                   kPerChannel ? (static_cast<float>(acc[t][r][i]) * ws[t][0]) * sm
-                                               : y[t][r][i] * sm);
+                store_route_output(dst + 16u * t, (static_cast<float>(acc[t][r][i]) * ws[t]) * sm);
         }
 }
 
-template <uint32_t H, uint32_t I, uint32_t kWaves, uint32_t kTilesPerWave,
-          uint32_t kBlocksPerGroup, bool kBf16>
+template <uint32_t H, uint32_t I, uint32_t kWaves, uint32_t kTilesPerWave, bool kBf16>
 __global__ __launch_bounds__(kWaves * 64) void down_w8_wide_kernel(
     const uint4* __restrict__ w, const uint16_t* __restrict__ s,
     const int8_t* __restrict__ mq, const float* __restrict__ ms,
-    const q38m_task_v1* __restrict__ tasks, const uint32_t* __restrict__ live_tasks, float* __restrict__ out) {
+    const q38m_task_v1* __restrict__ tasks, uint32_t task_slots, float* __restrict__ out) {
     constexpr uint32_t kBlocks = I / 64u;
     constexpr uint32_t kTiles = H / 16u;
     constexpr uint32_t kThreads = kWaves * 64u;
@@ -1244,7 +744,7 @@ __global__ __launch_bounds__(kWaves * 64) void down_w8_wide_kernel(
     __shared__ float row_scale[kWideRows];
 
     Placement at;
-    if (!place_on_xcds(live_tasks, at)) return;
+    if (!place_on_xcds(task_slots, H / 16u / (kWaves * kTilesPerWave), at)) return;
     const TaskRecord task = read_task(tasks, at.task);
     const uint32_t rows = task.rows;
     if (rows == 0u) return;
@@ -1280,184 +780,10 @@ __global__ __launch_bounds__(kWaves * 64) void down_w8_wide_kernel(
         row_scale[threadIdx.x] = threadIdx.x < rows ? ms[p0 + threadIdx.x] : 0.0f;
     __syncthreads();
 
-    const uint16_t* ws_expert = s + static_cast<size_t>(e) * H * (kBlocks / kBlocksPerGroup);
+    const uint16_t* ws_expert = s + static_cast<size_t>(e) * H;
     auto run = [&](auto row_tiles) {
-        down_w8_wide_rows<H, I, kTilesPerWave, decltype(row_tiles)::value, kBlocksPerGroup,
-                          kBf16>(wt, ws_expert, a_lds, row_scale, rows, p0, tile0, out);
-    };
-    if (tiles > 4u)
-        run(std::integral_constant<uint32_t, 8>{});
-    else if (tiles > 2u)
-        run(std::integral_constant<uint32_t, 4>{});
-    else if (tiles == 2u)
-        run(std::integral_constant<uint32_t, 2>{});
-    else
-        run(std::integral_constant<uint32_t, 1>{});
-}
-
-// Down, W4 group-32 (the all-W4 layer policy), over a task of up to 128
-// rows: the gate/up chain over K = I.  The mid rows are staged once in LDS
-// as [group][row tile][lane] 8-byte fragments; a workgroup of 16 waves
-// covers 32 output tiles, two per wave, kStride tiles apart: the two
-// 64-byte halves of an output line come from neighbouring waves at about
-// the same time and meet in L2 (adjacent tiles in one wave were stored a
-// whole tile's chain apart, and 9 % of the route-output bytes went to HBM
-// twice).  A wave streams its tiles' weights
-// one quad ahead and runs the chain group by group with the
-// same pinned MFMA/v_cvt/v_fma interleave as the gate/up kernel, over kRows
-// (8, 4, 2 or 1) row tiles picked per task; groups of 64 or 128 columns
-// chain their sub-blocks' int32 tiles as the gate/up kernel does.
-template <uint32_t H, uint32_t I, uint32_t kTilesPerWave, uint32_t kStride, uint32_t kRows,
-          uint32_t kSub, bool kBf16>
-__device__ __forceinline__ void down_w4_wide_rows(const uint4* __restrict__ wt,
-                                                  const uint16_t* __restrict__ st,
-                                                  const uint2* a_lds, const float* row_scale,
-                                                  uint32_t rows, uint32_t p0, uint32_t tile0,
-                                                  float* __restrict__ out) {
-    constexpr uint32_t kQuads = I / 128u;
-    constexpr uint32_t kTiles = H / 16u;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t n = lane & 15u;
-    const uint32_t q = lane >> 4;
-    const uint2* abuf = a_lds + lane;
-    const v4i zero = {0, 0, 0, 0};
-    // quad-major layout: quad kq of tile t is unit kq*kTiles + t of the
-    // expert; weights stream one quad ahead, across tile boundaries too
-    auto load = [&](uint32_t t, uint32_t kq) {
-        const uint32_t tt = t < kTilesPerWave ? t : kTilesPerWave - 1u;
-        return TileQuad{wt[(kq * kTiles + tt * kStride) * 64u],
-                        load_quad_scales<kSub, false>(st + (kq * kTiles + tt * kStride) * 16u *
-                                                               (4u / kSub))};
-    };
-    TileQuad cur = load(0, 0);
-#pragma unroll 1
-    for (uint32_t t = 0; t < kTilesPerWave; ++t) {
-        float y[kRows][4];
-#pragma unroll
-        for (uint32_t r = 0; r < kRows; ++r)
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i) y[r][i] = 0.0f;
-#pragma unroll 1
-        for (uint32_t kq = 0; kq < kQuads; ++kq) {
-          const TileQuad next = kq + 1u < kQuads ? load(t, kq + 1u) : load(t + 1u, 0);
-          const uint32_t bw[4] = {cur.w.x, cur.w.y, cur.w.z, cur.w.w};
-          v4i chain[kRows];  // kSub > 1: the group's running int32 tiles
-#pragma unroll
-          for (uint32_t j = 0; j < 4u; ++j) {
-            const uint32_t g = kq * 4u + j;
-            long a[kRows];
-#pragma unroll
-            for (uint32_t r = 0; r < kRows; ++r) a[r] = as_long(abuf[(g * kRowTiles + r) * 64u]);
-            const long bj = unpack_w4x16(bw[j]);
-            if (j % kSub != kSub - 1u) {
-#pragma unroll
-              for (uint32_t r = 0; r < kRows; ++r)
-                chain[r] = mfma_i8_16x16x32(a[r], bj, j % kSub == 0u ? zero : chain[r]);
-              continue;
-            }
-            const uint32_t word = quad_scale_word(cur.s, j / kSub);
-            const float scale = (kBf16 ? bf16_to_f32(word) : f16_to_f32(word)) * 0.0625f;
-            // the group's int32 tile r: d[r & 1] (kSub == 1) or chain[r] in place
-            v4i d[2];
-            auto issue = [&](uint32_t r) {
-                if constexpr (kSub == 1u) d[r & 1u] = mfma_i8_16x16x32(a[r], bj, zero);
-                else chain[r] = mfma_i8_16x16x32(a[r], bj, chain[r]);
-            };
-            auto tile = [&](uint32_t r) -> const v4i& {
-                if constexpr (kSub == 1u) return d[r & 1u];
-                else return chain[r];
-            };
-            issue(0);
-#pragma unroll
-            for (uint32_t r = 0; r < kRows; ++r) {
-                if (r + 1u < kRows) issue(r + 1u);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    y[r][i] = __builtin_fmaf(static_cast<float>(tile(r)[i]), scale, y[r][i]);
-                asm volatile("" : "+v"(y[r][0]), "+v"(y[r][1]), "+v"(y[r][2]), "+v"(y[r][3]));
-                __builtin_amdgcn_sched_barrier(0);
-            }
-          }
-          cur = next;
-        }
-        const uint32_t channel = (tile0 + t * kStride) * 16u + n;
-        // re-derived in every tile, so the 32 output addresses are not
-        // hoisted out of the tile loop into registers
-        uint32_t lane_row = 4u * q;
-        asm volatile("" : "+v"(lane_row));
-#pragma unroll
-        for (uint32_t r = 0; r < kRows; ++r)
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i) {
-                const uint32_t row = 16u * r + lane_row + i;
-                if (row >= rows) continue;
-                store_route_output(out + static_cast<size_t>(p0 + row) * H + channel,
-                                   y[r][i] * row_scale[row]);
-            }
-    }
-}
-
-template <uint32_t H, uint32_t I, uint32_t kWaves, uint32_t kTilesPerWave, uint32_t kSub,
-          bool kBf16>
-__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4)))
-void down_w4_wide_kernel(
-    const uint4* __restrict__ w, const uint16_t* __restrict__ s,
-    const int8_t* __restrict__ mq, const float* __restrict__ ms,
-    const q38m_task_v1* __restrict__ tasks, const uint32_t* __restrict__ live_tasks, float* __restrict__ out) {
-    constexpr uint32_t kQuads = I / 128u;
-    constexpr uint32_t kGroups = I / 32u;
-    constexpr uint32_t kTiles = H / 16u;
-    constexpr uint32_t kThreads = kWaves * 64u;
-    constexpr uint32_t kPieces = kWideRows * (I / 16u);
-    static_assert(kPieces % kThreads == 0u, "whole pieces per thread");
-    __shared__ uint2 a_lds[kGroups * kRowTiles * 64u];
-    __shared__ float row_scale[kWideRows];
-
-    Placement at;
-    if (!place_on_xcds(live_tasks, at)) return;
-    const TaskRecord task = read_task(tasks, at.task);
-    const uint32_t rows = task.rows;
-    if (rows == 0u) return;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t n = lane & 15u;
-    const uint32_t e = task.expert;
-    const uint32_t p0 = task.begin;
-
-    // Piece i: row r, 16-byte piece c = group c/2, lane groups 2(c%2),
-    // 2(c%2)+1; all loads before the first store.
-    constexpr uint32_t kPer = kPieces / kThreads;
-    uint4 v[kPer];
-#pragma unroll
-    for (uint32_t u = 0; u < kPer; ++u) {
-        const uint32_t i = threadIdx.x + u * kThreads;
-        const uint32_t r = i / (I / 16u), c = i % (I / 16u);
-        v[u] = reinterpret_cast<const uint4*>(mq + static_cast<size_t>(p0 + (r < rows ? r : 0u)) *
-                                                       I)[c];
-    }
-#pragma unroll
-    for (uint32_t u = 0; u < kPer; ++u) {
-        const uint32_t i = threadIdx.x + u * kThreads;
-        const uint32_t r = i / (I / 16u), c = i % (I / 16u);
-        const uint4 x = r < rows ? v[u] : make_uint4(0u, 0u, 0u, 0u);
-        const uint32_t at = ((c >> 1) * kRowTiles + r / 16u) * 64u + (c & 1u) * 32u + r % 16u;
-        a_lds[at] = make_uint2(x.x, x.y);
-        a_lds[at + 16u] = make_uint2(x.z, x.w);
-    }
-    if (threadIdx.x < kWideRows)
-        row_scale[threadIdx.x] = threadIdx.x < rows ? ms[p0 + threadIdx.x] : 0.0f;
-    __syncthreads();
-
-    // wave w: tiles tile0 + t * kWaves
-    const uint32_t tile0 = at.slice * kWaves * kTilesPerWave + wave;
-    const uint4* wt = w + (static_cast<size_t>(e) * kQuads * kTiles + tile0) * 64u + lane;
-    const uint16_t* st =
-        s + ((static_cast<size_t>(e) * kQuads * kTiles + tile0) * 16u + n) * (4u / kSub);
-    const uint32_t tiles = (rows + 15u) / 16u;  // uniform per workgroup
-    auto run = [&](auto row_tiles) {
-        down_w4_wide_rows<H, I, kTilesPerWave, kWaves, decltype(row_tiles)::value, kSub, kBf16>(
-            wt, st, a_lds, row_scale, rows, p0, tile0, out);
+        down_w8_wide_rows<H, I, kTilesPerWave, decltype(row_tiles)::value, kBf16>(
+            wt, ws_expert, a_lds, row_scale, rows, p0, tile0, out);
     };
     if (tiles > 4u)
         run(std::integral_constant<uint32_t, 8>{});
@@ -1484,7 +810,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
 void down_w4g32_f16_kernel(const uint4* __restrict__ w, const uint16_t* __restrict__ s,
                            const int8_t* __restrict__ mq, const float* __restrict__ ms,
                            const q38m_task_v1* __restrict__ tasks,
-                           const uint32_t* __restrict__ live_tasks, float* __restrict__ out) {
+                           uint32_t task_slots, float* __restrict__ out) {
     constexpr uint32_t kSteps = I / 64u;
     constexpr uint32_t kTiles = H / 16u;
     static_assert(kSteps % 2u == 0u, "steps run in pairs of LDS buffers");
@@ -1492,7 +818,7 @@ void down_w4g32_f16_kernel(const uint4* __restrict__ w, const uint16_t* __restri
     __shared__ float row_scale[kWideRows];
 
     Placement at;
-    if (!place_on_xcds(live_tasks, at)) return;
+    if (!place_on_xcds(task_slots, H / 16u / 16u, at)) return;
     const TaskRecord task = read_task(tasks, at.task);
     const uint32_t rows = task.rows;
     if (rows == 0u) return;
@@ -1652,6 +978,351 @@ void down_w4g32_f16_kernel(const uint4* __restrict__ w, const uint16_t* __restri
     }
 }
 
+// ---- gate/up and down on 32x32 int8 MFMA ------------------------------------
+//
+// Every chunk format whose scale groups are at least 64 columns wide (W4 in
+// groups of 64 or 128, W8 in groups of 64 or 128, W8 per channel for
+// gate/up) runs one kernel.  A workgroup of four waves covers eight adjacent
+// weight slots (128 output channels) and 64 rows of one task; wave w owns
+// slots 2w and 2w + 1 -- the gate and the up tile of a channel pair, or two
+// adjacent output tiles of down -- as the 32 columns of
+// v_mfma_i32_32x32x32_i8, over one or two 32-row tiles.  Per 128-column step
+// the workgroup stages its int8 rows in a double-buffered 8 KB LDS image;
+// a wave's weights go straight to its registers, one to three steps ahead.
+//
+// What bounds it: the matrix cores and the VALU take turns on this part (a
+// microbenchmark of the two mixed at four VALU instructions per MFMA or more
+// takes the sum of their times), so a step costs its MFMAs plus its VALU
+// instructions.  The 32x32 form does twice the work of the 16x16x32 form
+// per matrix cycle and leaves a quarter of its cycles to the VALU.  The
+// group chain is two VALU instructions per element: the MFMA accumulator
+// starts from the bits of 1.5 * 2^23, so its result read as a float is
+// 12582912 + acc exactly (|acc| < 2^22: 16 w a over 128 columns stays below
+// 2.1e6), one v_add_f32 recovers (float)acc -- v_cvt_f32_i32 runs at half
+// rate -- and one v_fma_f32 continues y = fmaf((float)acc_g, s_g, y) in group
+// order.  W4 nibbles sit in the high half of their byte (16 w), so their
+// scale is s / 16, exact.  Measured against the 16x16 kernels it replaces
+// (128-row tasks, 16 waves): W4 groups of 128 at 6,001 tokens gate/up 411 ->
+// 300 us and down 300 -> 208 us (down's 491 MB of route outputs alone: 97 us);
+// W8 groups of 128 at 1,500 tokens 285 -> 190 and 136 -> 110 us, at 8,192
+// tokens 751 -> 501 and 424 -> 334 us.  64 rows per workgroup at three waves
+// per SIMD run as fast as 128 rows at two (W8 181 / 113 us, W4 330 / 250);
+// rows resident in LDS over all of K with one workgroup per CU take 384-469
+// us for the W4 gate/up, non-temporal weights 337 us.
+//
+// A image: row r's 16-byte chunk c (0..7 of the step's 128 columns) is at
+// slot c * 64 + (r ^ c): the staging stores (eight chunks of a row by eight
+// neighbouring lanes) and the fragment reads (one chunk, 32 rows) both fall
+// in distinct banks.  MFMA j of a step takes chunks 2j and 2j + 1, lane
+// (h, r) row r of chunk 2j + h; the weights' lane (h, c) brings column c's
+// same 16 values: words j of lanes (2h, n) and (2h + 1, n) of a W4 quad, or
+// the 16 bytes of lane q = 2 (j % 2) + h of a W8 64-column block j / 2.
+constexpr uint32_t kI8Rows = 64;  // rows per workgroup
+
+template <uint32_t kBits, uint32_t kGroup, bool kGateUp>
+struct WideI8 {
+    static constexpr uint32_t kK = kGateUp ? kHidden : kInter;
+    static constexpr uint32_t kSlots = kGateUp ? 2u * kInter / 16u : kHidden / 16u;
+    static constexpr uint32_t kSteps = kK / 128u;
+    static constexpr uint32_t kSlices = kSlots / 8u;  // workgroups per 64 rows of a task
+    static constexpr uint32_t kHalves = kWideRows / kI8Rows;
+    static constexpr bool kPerChannel = kGroup == 0u;
+    static constexpr uint32_t kGroups = kGroup == 64u ? 2u : 1u;  // chain steps per 128 columns
+    static constexpr uint32_t kMfma = 4u / kGroups;               // MFMAs per chain step
+    static constexpr uint32_t kLoads = kBits == 4u ? 2u : 4u;     // 16-byte weight loads per step
+};
+
+template <uint32_t kBits, uint32_t kGroup, bool kBf16, bool kGateUp>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+void wide_i8_kernel(const uint4* __restrict__ w, const uint16_t* __restrict__ s,
+                    const int8_t* __restrict__ rows_q, const float* __restrict__ row_scales,
+                    const uint32_t* __restrict__ packed, const float* __restrict__ route_weights,
+                    const q38m_task_v1* __restrict__ tasks, uint32_t task_slots, void* __restrict__ out) {
+    using F = WideI8<kBits, kGroup, kGateUp>;
+    constexpr uint32_t kK = F::kK, kSlots = F::kSlots, kSteps = F::kSteps;
+    static_assert(kSteps % 2u == 0u, "steps run in pairs of LDS buffers");
+    static_assert(kBits == 8u || kGroup != 0u, "W4 is always grouped");
+    __shared__ u32x4 a_lds[2][8u * kI8Rows];
+    __shared__ float2 row_info[kI8Rows];  // (row scale, route weight)
+
+    Placement at;
+    if (!place_on_xcds(task_slots, F::kSlices * F::kHalves, at)) return;
+    const TaskRecord task = read_task(tasks, at.task);
+    // this workgroup's rows of the task: 64 from row 64 * half
+    const uint32_t half = at.slice / F::kSlices;
+    const uint32_t slice = at.slice % F::kSlices;
+    if (task.rows <= kI8Rows * half) return;
+    const uint32_t rows = min(task.rows - kI8Rows * half, kI8Rows);
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t c = lane & 31u, h = lane >> 5, n = lane & 15u;
+    const uint32_t e = task.expert;
+    const uint32_t p0 = task.begin + kI8Rows * half;
+    const uint32_t slot0 = slice * 8u + 2u * wave;
+    const uint32_t slot = slot0 + (c >> 4);
+
+    // staging: pieces u = 0, 1, row tid/8 + 32u, 16-byte chunk tid%8; a row
+    // past the task reads a row that exists, and its products land in rows
+    // that are never stored
+    const uint32_t sch = tid & 7u;
+    uint32_t a_off[2];
+#pragma unroll
+    for (uint32_t u = 0; u < 2u; ++u) {
+        const uint32_t r = (tid >> 3) + 32u * u;
+        if constexpr (kGateUp) {
+            uint32_t token = 0u;
+            if (r < rows) {
+                const uint32_t a = checked(packed[p0 + r], Q38M_WIDE_MAX_TOKENS * kTopK, kCheckToken);
+                token = a / kTopK;
+                if (sch == 0u) row_info[r] = make_float2(row_scales[token], route_weights[a]);
+            }
+            a_off[u] = token * kK + sch * 16u;
+        } else {
+            a_off[u] = (p0 + (r < rows ? r : 0u)) * kK + sch * 16u;
+            if (sch == 0u && r < rows) row_info[r] = make_float2(row_scales[p0 + r], 0.0f);
+        }
+    }
+    const uint32_t a_at = sch * kI8Rows + ((tid >> 3) ^ sch);
+
+    // the wave's weights: see the layouts in q38m.h
+    const uint4* w_step;  // uniform, advanced per step
+    uint32_t w_off;       // the lane's 16-byte piece of load 0
+    constexpr uint32_t kWStep = kBits == 4u ? kSlots * 64u : kGateUp ? 2u * kSlots * 64u : 128u;
+    if constexpr (kBits == 4u) {
+        w_step = w + static_cast<size_t>(e) * kSteps * kSlots * 64u;
+        w_off = slot * 64u + 32u * h + n;
+    } else if constexpr (kGateUp) {
+        w_step = w + static_cast<size_t>(e) * (kK / 64u) * kSlots * 64u;
+        w_off = slot * 64u + 16u * h + n;
+    } else {
+        w_step = w + static_cast<size_t>(e) * (kK / 64u) * kSlots * 64u;
+        w_off = slot * (kK / 64u) * 64u + 16u * h + n;
+    }
+    const uint16_t* s_base;  // the lane's scale words of step 0
+    constexpr uint32_t kSStep =
+        kBits == 4u ? kSlots * 16u * F::kGroups : F::kPerChannel ? 0u : F::kGroups;
+    if constexpr (kBits == 4u) {
+        s_base = s + ((static_cast<size_t>(e) * kSteps * kSlots + slot) * 16u + n) * F::kGroups;
+    } else {
+        const uint32_t row = kGateUp ? (c >> 4) * kInter + (slot0 >> 1) * 16u + n : slot * 16u + n;
+        const uint32_t per_row = F::kPerChannel ? 1u : kK / 128u * F::kGroups;
+        s_base = s + (static_cast<size_t>(e) * kSlots * 16u + row) * per_row;
+    }
+    struct Weights {
+        u32x4 v[F::kLoads];
+        uint32_t s;
+    };
+    auto load_weights = [&](uint32_t step) __attribute__((always_inline)) {
+        Weights x;
+        const u32x4* p = reinterpret_cast<const u32x4*>(w_step) + static_cast<size_t>(step) * kWStep;
+#pragma unroll
+        for (uint32_t j = 0; j < F::kLoads; ++j) {
+            constexpr uint32_t kBlock = kGateUp ? kSlots * 64u : 64u;  // W8: the next 64 columns
+            x.v[j] = p[w_off + (kBits == 4u ? 16u * j : (j >> 1) * kBlock + (j & 1u) * 32u)];
+        }
+        const uint16_t* q = s_base + static_cast<size_t>(step) * kSStep;
+        if constexpr (F::kGroups == 2u) x.s = *reinterpret_cast<const uint32_t*>(q);
+        else x.s = *q;
+        return x;
+    };
+
+    v16i bias;
+#pragma unroll
+    for (uint32_t i = 0; i < 16u; ++i) bias[i] = F::kPerChannel ? 0 : 0x4B400000;
+    if constexpr (!F::kPerChannel) asm volatile("" : "+v"(bias));  // one register block
+    float unbias;  // -12582912.0f in a scalar register (no literal per use)
+    asm volatile("s_mov_b32 %0, 0xcb400000" : "=s"(unbias));
+    auto lds_barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+
+    auto run = [&](auto row_tiles) __attribute__((always_inline)) {
+        constexpr uint32_t kNt = decltype(row_tiles)::value;
+        float y[kNt][16];  // grouped: the fp32 chain
+        v16i acc[F::kPerChannel ? kNt : 1];
+#pragma unroll
+        for (uint32_t t = 0; t < kNt; ++t)
+#pragma unroll
+            for (uint32_t i = 0; i < 16u; ++i) y[t][i] = 0.0f;
+        if constexpr (F::kPerChannel) {
+#pragma unroll
+            for (uint32_t t = 0; t < kNt; ++t) acc[t] = bias;
+        }
+        struct Rows {
+            u32x4 v[kNt];
+        };
+        auto load_rows = [&](uint32_t step) __attribute__((always_inline)) {
+            Rows x;
+            const int8_t* p = rows_q + step * 128u;
+#pragma unroll
+            for (uint32_t u = 0; u < kNt; ++u) x.v[u] = *reinterpret_cast<const u32x4*>(p + a_off[u]);
+            return x;
+        };
+        auto store_rows = [&](const Rows& x, uint32_t buffer) __attribute__((always_inline)) {
+#pragma unroll
+            for (uint32_t u = 0; u < kNt; ++u) a_lds[buffer][a_at + 32u * u] = x.v[u];
+        };
+        // weights in flight: one step (two row tiles) or three (one tile,
+        // whose steps are short against the memory latency); W4 sets are
+        // unpacked at the start of their step and refilled at once
+        constexpr uint32_t kRing = kBits == 4u ? (kNt == 1u ? 4u : 1u) : (kNt == 1u ? 4u : 2u);
+        Weights ring[kRing];
+        Rows ahead;
+        auto clamped = [](uint32_t k) { return k < kSteps ? k : kSteps - 1u; };
+
+        // step k on LDS buffer j4 % 2 (j4 = k % 4, a compile-time constant)
+        auto step = [&](uint32_t k, auto jc) __attribute__((always_inline)) {
+            constexpr uint32_t j4 = decltype(jc)::value;
+            constexpr uint32_t buffer = j4 & 1u;
+            ahead = load_rows(clamped(k + 1u));
+            if constexpr (kBits == 8u) ring[(j4 + kRing - 1u) % kRing] = load_weights(clamped(k + kRing - 1u));
+            const Weights& x = ring[j4 % kRing];
+            v4i b[4];
+            float sc[F::kGroups];
+            if constexpr (kBits == 4u) {
+                const uint32_t lo[4] = {x.v[0].x, x.v[0].y, x.v[0].z, x.v[0].w};
+                const uint32_t hi[4] = {x.v[1].x, x.v[1].y, x.v[1].z, x.v[1].w};
+#pragma unroll
+                for (uint32_t j = 0; j < 4u; ++j) {
+                    b[j].x = static_cast<int>((lo[j] << 4) & 0xf0f0f0f0u);
+                    b[j].y = static_cast<int>(lo[j] & 0xf0f0f0f0u);
+                    b[j].z = static_cast<int>((hi[j] << 4) & 0xf0f0f0f0u);
+                    b[j].w = static_cast<int>(hi[j] & 0xf0f0f0f0u);
+                }
+            } else {
+#pragma unroll
+                for (uint32_t j = 0; j < 4u; ++j) b[j] = __builtin_bit_cast(v4i, x.v[j]);
+            }
+#pragma unroll
+            for (uint32_t g = 0; g < F::kGroups; ++g) {
+                const uint32_t word = (x.s >> (16u * g)) & 0xffffu;
+                sc[g] = (kBf16 ? bf16_to_f32(word) : f16_to_f32(word)) * (kBits == 4u ? 0.0625f : 1.0f);
+                asm volatile("" : "+v"(sc[g]));  // a plain v_fma_f32, not v_fma_mix
+            }
+            if constexpr (kBits == 4u) {
+                __builtin_amdgcn_sched_barrier(0);
+                ring[j4 % kRing] = load_weights(clamped(k + kRing));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const u32x4* image = a_lds[buffer] + h * kI8Rows;
+            auto fragment = [&](uint32_t t, uint32_t j) __attribute__((always_inline)) {
+                return __builtin_bit_cast(v4i, image[2u * j * kI8Rows + 32u * t + (c ^ (2u * j + h))]);
+            };
+            // kBatch fragments at a time: MFMA batch q of tile t is MFMAs
+            // kBatch q .. kBatch q + kBatch - 1, the next batch's fragments
+            // requested behind it
+            constexpr uint32_t kBatch = kGateUp ? F::kMfma : 2u;
+            constexpr uint32_t kBatches = 4u / kBatch;
+            v4i fa[kBatch];
+#pragma unroll
+            for (uint32_t i = 0; i < kBatch; ++i) fa[i] = fragment(0u, i);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (uint32_t t = 0; t < kNt; ++t) {
+                v16i& d = acc[F::kPerChannel ? t : 0u];
+#pragma unroll
+                for (uint32_t q = 0; q < kBatches; ++q) {
+#pragma unroll
+                    for (uint32_t i = 0; i < kBatch; ++i) {
+                        const uint32_t j = q * kBatch + i;
+                        d = mfma_i8_32x32x32(fa[i], b[j], !F::kPerChannel && j % F::kMfma == 0u ? bias : d);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    const uint32_t next = t * kBatches + q + 1u;
+                    if (next < kNt * kBatches) {
+#pragma unroll
+                        for (uint32_t i = 0; i < kBatch; ++i)
+                            fa[i] = fragment(next / kBatches, next % kBatches * kBatch + i);
+                    }
+                    if constexpr (!F::kPerChannel) {
+                        if ((q + 1u) * kBatch % F::kMfma == 0u) {
+                            const uint32_t g = ((q + 1u) * kBatch - 1u) / F::kMfma;
+#pragma unroll
+                            for (uint32_t i = 0; i < 16u; ++i)
+                                y[t][i] = __builtin_fmaf(__int_as_float(d[i]) + unbias, sc[g], y[t][i]);
+#pragma unroll
+                            for (uint32_t i = 0; i < 16u; i += 4u)
+                                asm volatile("" : "+v"(y[t][i]), "+v"(y[t][i + 1u]), "+v"(y[t][i + 2u]),
+                                             "+v"(y[t][i + 3u]));
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            store_rows(ahead, buffer ^ 1u);
+            lds_barrier();
+        };
+        // before step 0: its rows in buffer 0, the first steps' weights in
+        // flight; loads past the end repeat the last step's, unread
+        static_assert(kSteps % 4u == 0u, "the loop covers four ring slots");
+#pragma unroll
+        for (uint32_t j = 0; j + (kBits == 8u ? 1u : 0u) < kRing; ++j) ring[j] = load_weights(j);
+        ahead = load_rows(0u);
+        store_rows(ahead, 0u);
+        __syncthreads();
+#pragma unroll 1
+        for (uint32_t k = 0; k < kSteps; k += 4u) {
+            step(k, std::integral_constant<uint32_t, 0>{});
+            step(k + 1u, std::integral_constant<uint32_t, 1>{});
+            step(k + 2u, std::integral_constant<uint32_t, 2>{});
+            step(k + 3u, std::integral_constant<uint32_t, 3>{});
+        }
+        if constexpr (F::kPerChannel) {
+            const float scale = kBf16 ? bf16_to_f32(ring[0].s) : f16_to_f32(ring[0].s);
+#pragma unroll
+            for (uint32_t t = 0; t < kNt; ++t)
+#pragma unroll
+                for (uint32_t i = 0; i < 16u; ++i) y[t][i] = static_cast<float>(acc[t][i]) * scale;
+        }
+
+        // D lane (h, c): column c, rows 8 (i/4) + 4h + i%4 of each tile
+        if constexpr (kGateUp) {
+            // lanes 0-15 of a half hold a channel's gate values, lanes 16-31
+            // its up values: exchanging two elements' halves leaves every
+            // lane one element's gate and up
+            uint16_t* mid = static_cast<uint16_t*>(out);
+            const uint32_t channel = (slot0 >> 1) * 16u + n;
+            const uint32_t odd = (lane >> 4) & 1u;
+#pragma unroll
+            for (uint32_t t = 0; t < kNt; ++t) {
+                uint32_t silu_word[8];
+                float up_value[8];
+#pragma unroll
+                for (uint32_t i = 0; i < 16u; i += 2u) {
+                    const uint32_t r = 32u * t + 8u * (i / 4u) + 4u * h + i % 4u + odd;
+                    const auto pair = __builtin_amdgcn_permlane16_swap(
+                        __float_as_uint(y[t][i]), __float_as_uint(y[t][i + 1u]), false, false);
+                    const float st = row_info[r < rows ? r : 0u].x;
+                    up_value[i / 2u] = bf16_round(__uint_as_float(pair[1]) * st);
+                    silu_word[i / 2u] = kSiluTable[f32_to_bf16(__uint_as_float(pair[0]) * st)];
+                }
+#pragma unroll
+                for (uint32_t i = 0; i < 16u; i += 2u) {
+                    const uint32_t r = 32u * t + 8u * (i / 4u) + 4u * h + i % 4u + odd;
+                    if (r >= rows) continue;
+                    const float hv = bf16_round(__uint_as_float(silu_word[i / 2u]) * up_value[i / 2u]);
+                    mid[static_cast<size_t>(p0 + r) * kInter + channel] = static_cast<uint16_t>(
+                        bf16_canonical_nan(f32_to_bf16(hv * row_info[r].y)));
+                }
+            }
+        } else {
+            float* route = static_cast<float*>(out) + slot0 * 16u + c;
+#pragma unroll
+            for (uint32_t t = 0; t < kNt; ++t)
+#pragma unroll
+                for (uint32_t i = 0; i < 16u; ++i) {
+                    const uint32_t r = 32u * t + 8u * (i / 4u) + 4u * h + i % 4u;
+                    if (r >= rows) continue;
+                    store_route_output(route + static_cast<size_t>(p0 + r) * kHidden,
+                                       y[t][i] * row_info[r].x);
+                }
+        }
+    };
+    if (rows > 32u)
+        run(std::integral_constant<uint32_t, 2>{});
+    else
+        run(std::integral_constant<uint32_t, 1>{});
+}
+
 }  // namespace
 
 uint32_t wide_chunks(uint32_t tokens) {
@@ -1672,83 +1343,31 @@ hipError_t launch_build_wide_plan(const int32_t* ids, uint32_t tokens,
 
 namespace {
 
-// the task slots a launch covers: grid rows, and the device word with the
-// number the plan filled
+// the task slots a launch covers
 struct TaskSlots {
     const q38m_task_v1* tasks;
-    const uint32_t* live;
     uint32_t count;
 };
 
-template <uint32_t kSub, bool kBf16>
-void launch_gate_up_wide_sub(const q38m_expert_weights_v1& w, const int8_t* xq, const float* xs,
-                             const uint32_t* packed, const float* route_weights,
-                             const TaskSlots& t, uint16_t* weighted_mid, hipStream_t stream) {
-    if constexpr (kSub == 1u) {
-        // fp16 MFMA form: 8 channel pairs (256 rows of gate/up) per workgroup
-        const dim3 grid(kInter / 16u / 8u, t.count);
-        gate_up_w4g32_f16_kernel<kHidden, kInter, kBf16>
-            <<<grid, 512, 0, stream>>>(static_cast<const uint4*>(w.data),
-                                        static_cast<const uint16_t*>(w.scales), xq, xs, packed,
-                                        route_weights, t.tasks, t.live, weighted_mid);
-        return;
-    }
-    // 8 channel pairs (256 rows of gate/up) per workgroup
-    const dim3 grid(kInter / 16u / 8u, t.count);
-    gate_up_w4_wide_kernel<kHidden, kInter, kSub, kBf16>
-        <<<grid, 1024, 0, stream>>>(static_cast<const uint4*>(w.data),
-                                    static_cast<const uint16_t*>(w.scales), xq, xs, packed,
-                                    route_weights, t.tasks, t.live, weighted_mid);
+template <uint32_t kBits, uint32_t kGroup, bool kBf16>
+void launch_gate_up_i8(const q38m_expert_weights_v1& w, const int8_t* xq, const float* xs,
+                       const uint32_t* packed, const float* route_weights, const TaskSlots& t,
+                       uint16_t* mid, hipStream_t stream) {
+    using F = WideI8<kBits, kGroup, true>;
+    const uint32_t grid = placed_workgroups(t.count, F::kSlices * F::kHalves);
+    wide_i8_kernel<kBits, kGroup, kBf16, true><<<grid, 256, 0, stream>>>(
+        static_cast<const uint4*>(w.data), static_cast<const uint16_t*>(w.scales), xq, xs, packed,
+        route_weights, t.tasks, t.count, mid);
 }
 
-// Per channel: four tiles per wave (the tuned BASELINE shape).  Grouped:
-// the fp32 chain doubles the live accumulator state, so one tile per wave.
-template <uint32_t kBlocksPerGroup, bool kBf16>
-void launch_down_w8_wide_groups(const q38m_expert_weights_v1& w, const int8_t* mid_q,
-                                const float* mid_s, const TaskSlots& t, float* route_output,
-                                hipStream_t stream) {
-    constexpr uint32_t kWaves = 8;
-    constexpr uint32_t kTilesPerWave = kBlocksPerGroup == kInter / 64u ? 4u : 1u;
-    const dim3 grid(kHidden / 16u / (kWaves * kTilesPerWave), t.count);
-    down_w8_wide_kernel<kHidden, kInter, kWaves, kTilesPerWave, kBlocksPerGroup, kBf16>
-        <<<grid, kWaves * 64u, 0, stream>>>(static_cast<const uint4*>(w.data),
-                                            static_cast<const uint16_t*>(w.scales), mid_q, mid_s,
-                                            t.tasks, t.live, route_output);
-}
-
-template <uint32_t kSub, bool kBf16>
-void launch_down_w4_wide_sub(const q38m_expert_weights_v1& w, const int8_t* mid_q,
-                             const float* mid_s, const TaskSlots& t, float* route_output,
-                             hipStream_t stream) {
-    if constexpr (kSub == 1u) {
-        // fp16 MFMA form: 16 output tiles per 8-wave workgroup
-        const dim3 grid(kHidden / 16u / 16u, t.count);
-        down_w4g32_f16_kernel<kHidden, kInter, kBf16>
-            <<<grid, 512, 0, stream>>>(static_cast<const uint4*>(w.data),
-                                       static_cast<const uint16_t*>(w.scales), mid_q, mid_s,
-                                       t.tasks, t.live, route_output);
-        return;
-    }
-    constexpr uint32_t kWaves = 16, kTilesPerWave = 2;
-    const dim3 grid(kHidden / 16u / (kWaves * kTilesPerWave), t.count);
-    down_w4_wide_kernel<kHidden, kInter, kWaves, kTilesPerWave, kSub, kBf16>
-        <<<grid, kWaves * 64u, 0, stream>>>(static_cast<const uint4*>(w.data),
-                                            static_cast<const uint16_t*>(w.scales), mid_q, mid_s,
-                                            t.tasks, t.live, route_output);
-}
-
-template <uint32_t kBlocksPerGroup, bool kBf16>
-void launch_gate_up_w8_wide_groups(const q38m_expert_weights_v1& w, const int8_t* xq,
-                                   const float* xs, const uint32_t* packed,
-                                   const float* route_weights, const TaskSlots& t,
-                                   uint16_t* weighted_mid, hipStream_t stream) {
-    constexpr uint32_t kPairs = 8;
-    const dim3 grid(kInter / 16u / kPairs, t.count);
-    gate_up_w8_wide_kernel<kHidden, kInter, kPairs, kBlocksPerGroup, kBf16>
-        <<<grid, kPairs * 128u, 0, stream>>>(static_cast<const uint4*>(w.data),
-                                             static_cast<const uint16_t*>(w.scales), xq, xs,
-                                             packed, route_weights, t.tasks, t.live,
-                                             weighted_mid);
+template <uint32_t kBits, uint32_t kGroup, bool kBf16>
+void launch_down_i8(const q38m_expert_weights_v1& w, const int8_t* mid_q, const float* mid_s,
+                    const TaskSlots& t, float* route_output, hipStream_t stream) {
+    using F = WideI8<kBits, kGroup, false>;
+    const uint32_t grid = placed_workgroups(t.count, F::kSlices * F::kHalves);
+    wide_i8_kernel<kBits, kGroup, kBf16, false><<<grid, 256, 0, stream>>>(
+        static_cast<const uint4*>(w.data), static_cast<const uint16_t*>(w.scales), mid_q, mid_s,
+        nullptr, nullptr, t.tasks, t.count, route_output);
 }
 
 template <bool kBf16>
@@ -1756,28 +1375,21 @@ hipError_t launch_gate_up_wide_dtype(const q38m_expert_weights_v1& w, const int8
                                      const float* xs, const uint32_t* packed,
                                      const float* route_weights, const TaskSlots& t,
                                      uint16_t* mid, hipStream_t stream) {
-    if (w.format == Q38M_FORMAT_W8_SYM) {
-        switch (w.group_size) {
-            case 0u:
-                launch_gate_up_w8_wide_groups<kHidden / 64u, kBf16>(w, xq, xs, packed,
-                                                                    route_weights, t, mid, stream);
-                break;
-            case 64u:
-                launch_gate_up_w8_wide_groups<1, kBf16>(w, xq, xs, packed, route_weights, t, mid,
-                                                        stream);
-                break;
-            case 128u:
-                launch_gate_up_w8_wide_groups<2, kBf16>(w, xq, xs, packed, route_weights, t, mid,
-                                                        stream);
-                break;
-            default: return hipErrorInvalidValue;
+    const uint32_t key = (w.format == Q38M_FORMAT_W8_SYM ? 8000u : 4000u) + w.group_size;
+    switch (key) {
+        case 4032u: {
+            // fp16 MFMA form: 8 channel pairs (256 rows of gate/up) per workgroup
+            const uint32_t grid = placed_workgroups(t.count, kInter / 16u / 8u);
+            gate_up_w4g32_f16_kernel<kHidden, kInter, kBf16><<<grid, 512, 0, stream>>>(
+                static_cast<const uint4*>(w.data), static_cast<const uint16_t*>(w.scales), xq, xs,
+                packed, route_weights, t.tasks, t.count, mid);
+            break;
         }
-        return hipGetLastError();
-    }
-    switch (w.group_size) {
-        case 32u: launch_gate_up_wide_sub<1, kBf16>(w, xq, xs, packed, route_weights, t, mid, stream); break;
-        case 64u: launch_gate_up_wide_sub<2, kBf16>(w, xq, xs, packed, route_weights, t, mid, stream); break;
-        case 128u: launch_gate_up_wide_sub<4, kBf16>(w, xq, xs, packed, route_weights, t, mid, stream); break;
+        case 4064u: launch_gate_up_i8<4, 64, kBf16>(w, xq, xs, packed, route_weights, t, mid, stream); break;
+        case 4128u: launch_gate_up_i8<4, 128, kBf16>(w, xq, xs, packed, route_weights, t, mid, stream); break;
+        case 8000u: launch_gate_up_i8<8, 0, kBf16>(w, xq, xs, packed, route_weights, t, mid, stream); break;
+        case 8064u: launch_gate_up_i8<8, 64, kBf16>(w, xq, xs, packed, route_weights, t, mid, stream); break;
+        case 8128u: launch_gate_up_i8<8, 128, kBf16>(w, xq, xs, packed, route_weights, t, mid, stream); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1787,21 +1399,31 @@ template <bool kBf16>
 hipError_t launch_down_wide_dtype(const q38m_expert_weights_v1& w, const int8_t* mid_q,
                                   const float* mid_s, const TaskSlots& t, float* out,
                                   hipStream_t stream) {
-    constexpr uint32_t kBlocks = kInter / 64u;
-    if (w.format == Q38M_FORMAT_W8_SYM) {
-        switch (w.group_size) {
-            case 0u: launch_down_w8_wide_groups<kBlocks, kBf16>(w, mid_q, mid_s, t, out, stream); break;
-            case 64u: launch_down_w8_wide_groups<1, kBf16>(w, mid_q, mid_s, t, out, stream); break;
-            case 128u: launch_down_w8_wide_groups<2, kBf16>(w, mid_q, mid_s, t, out, stream); break;
-            default: return hipErrorInvalidValue;
+    const uint32_t key = (w.format == Q38M_FORMAT_W8_SYM ? 8000u : 4000u) + w.group_size;
+    switch (key) {
+        case 4032u: {
+            // fp16 MFMA form: 16 output tiles per 8-wave workgroup
+            const uint32_t grid = placed_workgroups(t.count, kHidden / 16u / 16u);
+            down_w4g32_f16_kernel<kHidden, kInter, kBf16><<<grid, 512, 0, stream>>>(
+                static_cast<const uint4*>(w.data), static_cast<const uint16_t*>(w.scales), mid_q,
+                mid_s, t.tasks, t.count, out);
+            break;
         }
-    } else {
-        switch (w.group_size) {
-            case 32u: launch_down_w4_wide_sub<1, kBf16>(w, mid_q, mid_s, t, out, stream); break;
-            case 64u: launch_down_w4_wide_sub<2, kBf16>(w, mid_q, mid_s, t, out, stream); break;
-            case 128u: launch_down_w4_wide_sub<4, kBf16>(w, mid_q, mid_s, t, out, stream); break;
-            default: return hipErrorInvalidValue;
+        case 4064u: launch_down_i8<4, 64, kBf16>(w, mid_q, mid_s, t, out, stream); break;
+        case 4128u: launch_down_i8<4, 128, kBf16>(w, mid_q, mid_s, t, out, stream); break;
+        case 8000u: {
+            // per channel: four tiles per wave
+            constexpr uint32_t kWaves = 8, kTilesPerWave = 4;
+            const uint32_t grid = placed_workgroups(t.count, kHidden / 16u / (kWaves * kTilesPerWave));
+            down_w8_wide_kernel<kHidden, kInter, kWaves, kTilesPerWave, kBf16>
+                <<<grid, kWaves * 64u, 0, stream>>>(static_cast<const uint4*>(w.data),
+                                                    static_cast<const uint16_t*>(w.scales), mid_q,
+                                                    mid_s, t.tasks, t.count, out);
+            break;
         }
+        case 8064u: launch_down_i8<8, 64, kBf16>(w, mid_q, mid_s, t, out, stream); break;
+        case 8128u: launch_down_i8<8, 128, kBf16>(w, mid_q, mid_s, t, out, stream); break;
+        default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
@@ -1810,9 +1432,8 @@ hipError_t launch_down_wide_dtype(const q38m_expert_weights_v1& w, const int8_t*
 
 hipError_t launch_gate_up_wide(const q38m_expert_weights_v1& w, const int8_t* xq, const float* xs,
                                const uint32_t* packed, const float* route_weights,
-                               const q38m_task_v1* tasks, const uint32_t* live_tasks,
-                               uint32_t task_count, uint16_t* weighted_mid, hipStream_t stream) {
-    const TaskSlots t{tasks, live_tasks, task_count};
+                               const q38m_task_v1* tasks, uint32_t task_count, uint16_t* weighted_mid, hipStream_t stream) {
+    const TaskSlots t{tasks, task_count};
     return w.scale_dtype == Q38M_SCALE_BF16
                ? launch_gate_up_wide_dtype<true>(w, xq, xs, packed, route_weights, t,
                                                  weighted_mid, stream)
@@ -1821,10 +1442,9 @@ hipError_t launch_gate_up_wide(const q38m_expert_weights_v1& w, const int8_t* xq
 }
 
 hipError_t launch_down_wide(const q38m_expert_weights_v1& w, const int8_t* mid_q,
-                            const float* mid_s, const q38m_task_v1* tasks,
-                            const uint32_t* live_tasks, uint32_t task_count,
+                            const float* mid_s, const q38m_task_v1* tasks, uint32_t task_count,
                             float* route_output, hipStream_t stream) {
-    const TaskSlots t{tasks, live_tasks, task_count};
+    const TaskSlots t{tasks, task_count};
     return w.scale_dtype == Q38M_SCALE_BF16
                ? launch_down_wide_dtype<true>(w, mid_q, mid_s, t, route_output, stream)
                : launch_down_wide_dtype<false>(w, mid_q, mid_s, t, route_output, stream);
