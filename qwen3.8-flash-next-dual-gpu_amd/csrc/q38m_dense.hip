@@ -27,8 +27,8 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
 constexpr uint32_t kDenseWaves = 4;
-// the 64 x 64 workgroup tile serves K up to this and grids of at least
-// this many tiles
+// one accumulator over K (64 x 64 workgroup tiles) for K up to this and grids
+// of at least this many tiles
 constexpr uint32_t kTile64MaxK = 1024;
 constexpr uint32_t kTile64MinTiles = 192;
 
@@ -580,6 +580,322 @@ __global__ __launch_bounds__(256) void shared_gate_up_kernel(
     }
 }
 
+// ---- large M: workgroup tiles of 64 or 128 rows and columns ----------------
+//
+// What bounds the 32 x 32 K-split tiles above once there are thousands of
+// activation rows is delivery from L2: every tile pulls its 64 rows over all
+// of K through its CU (4.2 GB for the router at 32,768 tokens).  Here a
+// workgroup of four waves owns a kTM x kTN tile, wave (wm, wn) its
+// (kTM/2) x (kTN/2) quarter over all of K, and each 64-wide K chunk of the
+// tile's kTM + kTN rows is staged once, by whole lines.  What bounds this
+// form is the latency of those loads, so they go straight to LDS
+// (global_load_lds_dwordx4, no registers) into a ring of kStages chunks:
+// kStages - 1 are in flight while one is multiplied, and the one barrier of
+// a step both publishes its chunk and retires the slot the next load fills.
+//
+// A load instruction of a wave fills eight rows of a slot, [row][8 x 16 B];
+// row r keeps its chunk c at position c ^ (r/2 % 8), so that fragment reads
+// (sixteen rows of one chunk) fall in distinct banks of the 256-byte LDS
+// row.  The lane that fills position p of row r reads chunk p ^ (r/2 % 8).
+//
+// The sums are those of the kernels above, bit for bit: kSplit, the four K
+// quarters' accumulators added in order (dense_gemm_kernel's waves);
+// otherwise one accumulator over all of K (dense_tile64_kernel's).
+//
+// The stacked B rows of a tile with kNB = 2 matrices are kTN/2 rows of the
+// first, then the same rows of the second, and a wave's columns are its
+// share of both.  With kGate the waves of column wn = 0 also multiply one
+// extra B row (gate_lds, all of K), as wave_partial does.
+template <uint32_t kTM_, uint32_t kTN_, uint32_t kNB_, uint32_t kStages_>
+struct TileShape {
+    static constexpr uint32_t kTM = kTM_, kTN = kTN_, kNB = kNB_, kStages = kStages_;
+    static constexpr uint32_t kRows = kTM + kTN;
+    static constexpr uint32_t kSlot = kRows * 8u;      // 16-byte vectors of a ring slot
+    static constexpr uint32_t kLoads = kRows / 32u;    // load instructions per wave and chunk
+    static constexpr uint32_t kI = kTM / 32u;          // a wave's row tiles
+    static constexpr uint32_t kJ = kTN / 32u / kNB;    // its column tiles per matrix
+    // all of a chunk's fragments in registers at once (beside 128 x 128 x 2
+    // matrices' accumulators and totals they would spill)
+    static constexpr bool kWholeChunk = kTM + kTN * kNB <= 256u;
+};
+
+// 16 bytes per lane from `src` (each lane its own) to the 1 KB at `lds`
+// (uniform), lane l at 16 l.  Counted by vmcnt like any load.
+__device__ __forceinline__ void load_to_lds(const u32x4* src, u32x4* lds) {
+    const uint32_t at = static_cast<uint32_t>(
+        reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) u32x4*)lds));
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src),
+                 "s"(__builtin_amdgcn_readfirstlane(at))
+                 : "memory", "m0");
+}
+
+// waits until at most kOutstanding of the wave's loads are in flight, then
+// for the workgroup's waves to get there; the wave's LDS reads are complete
+template <uint32_t kOutstanding>
+__device__ __forceinline__ void chunk_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(kOutstanding) : "memory");
+}
+
+template <typename S, bool kSplit, bool kGate, typename Finish>
+__device__ __forceinline__ void tile_product(const uint16_t* __restrict__ a,
+                                             const uint16_t* __restrict__ b0,
+                                             const uint16_t* __restrict__ b1, uint32_t m,
+                                             uint32_t n, uint32_t k, uint32_t m0, uint32_t n0,
+                                             u32x4* ring, const u32x4* gate_lds, Finish finish) {
+    constexpr uint32_t kTM = S::kTM, kTN = S::kTN, kNB = S::kNB, kStages = S::kStages;
+    constexpr uint32_t kI = S::kI, kJ = S::kJ, kLoads = S::kLoads;
+    const uint32_t t = threadIdx.x;
+    const uint32_t lane = t & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const uint32_t wm = wave >> 1, wn = wave & 1u;
+    // load i of the wave: stacked rows 8 (4 i + wave) + lane/8
+    const u32x4* src[kLoads];
+#pragma unroll
+    for (uint32_t i = 0; i < kLoads; ++i) {
+        const uint32_t row = 32u * i + 8u * wave + (lane >> 3);
+        const uint16_t* base;
+        if (32u * i < kTM) {
+            base = a + static_cast<size_t>(min(m0 + row, m - 1u)) * k;
+        } else {
+            const uint32_t r = row - kTM;
+            const bool second = kNB == 2u && 32u * i - kTM >= kTN / 2u;
+            base = (second ? b1 : b0) +
+                   static_cast<size_t>(min(n0 + (second ? r - kTN / 2u : r), n - 1u)) * k;
+        }
+        src[i] = reinterpret_cast<const u32x4*>(base) + ((lane & 7u) ^ ((row >> 1) & 7u));
+    }
+    auto load = [&](uint32_t c, uint32_t slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t i = 0; i < kLoads; ++i)
+            load_to_lds(src[i] + 8u * c, ring + slot * S::kSlot + (4u * i + wave) * 64u);
+    };
+    const uint32_t read_at = 8u * (lane & 15u);
+    const uint32_t swizzle = (lane >> 1) & 7u;
+    const uint32_t read_slot[2] = {read_at + ((lane >> 4) ^ swizzle),
+                                   read_at + ((4u + (lane >> 4)) ^ swizzle)};
+    const uint32_t a_row = 16u * kI * wm, b_row = kTM + 16u * kJ * wn;
+    const bool gate_lane = (lane & 15u) == 0u;
+    const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 acc[kNB][kI][kJ], total[kSplit ? kNB : 1][kSplit ? kI : 1][kSplit ? kJ : 1];
+    f32x4 acc_gate[kGate ? kI : 1], total_gate[kGate ? kI : 1];
+    auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t v = 0; v < kNB; ++v)
+#pragma unroll
+            for (uint32_t i = 0; i < kI; ++i)
+#pragma unroll
+                for (uint32_t j = 0; j < kJ; ++j) acc[v][i][j] = zero4;
+        if constexpr (kGate) {
+#pragma unroll
+            for (uint32_t i = 0; i < kI; ++i) acc_gate[i] = zero4;
+        }
+    };
+    // a K quarter is done: its sums join the earlier quarters'
+    auto fold = [&](bool first) __attribute__((always_inline)) {
+        if constexpr (kSplit) {
+#pragma unroll
+            for (uint32_t v = 0; v < kNB; ++v)
+#pragma unroll
+                for (uint32_t i = 0; i < kI; ++i)
+#pragma unroll
+                    for (uint32_t j = 0; j < kJ; ++j)
+                        total[v][i][j] = first ? acc[v][i][j] : total[v][i][j] + acc[v][i][j];
+            if constexpr (kGate) {
+#pragma unroll
+                for (uint32_t i = 0; i < kI; ++i)
+                    total_gate[i] = first ? acc_gate[i] : total_gate[i] + acc_gate[i];
+            }
+            clear();
+        }
+    };
+    auto multiply = [&](uint32_t c, uint32_t slot) __attribute__((always_inline)) {
+        // every fragment of the chunk is requested before its first MFMA (one
+        // exposed LDS latency a step; left to itself the compiler reads them
+        // a few at a time)
+        const u32x4* lds = ring + slot * S::kSlot;
+        u32x4 av[2][kI], bv[2][kNB][kJ], gv[2];
+        auto fragments = [&](uint32_t h) __attribute__((always_inline)) {
+#pragma unroll
+            for (uint32_t v = 0; v < kNB; ++v)
+#pragma unroll
+                for (uint32_t j = 0; j < kJ; ++j)
+                    bv[h][v][j] = lds[8u * (b_row + v * (kTN / 2u) + 16u * j) + read_slot[h]];
+#pragma unroll
+            for (uint32_t i = 0; i < kI; ++i) av[h][i] = lds[8u * (a_row + 16u * i) + read_slot[h]];
+            if constexpr (kGate) gv[h] = gate_lds[8u * c + 4u * h + (lane >> 4)];
+        };
+        if constexpr (S::kWholeChunk) {
+            fragments(0u);
+            fragments(1u);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (uint32_t h = 0; h < 2u; ++h) {
+            if constexpr (!S::kWholeChunk) fragments(h);
+#pragma unroll
+            for (uint32_t i = 0; i < kI; ++i)
+#pragma unroll
+                for (uint32_t v = 0; v < kNB; ++v)
+#pragma unroll
+                    for (uint32_t j = 0; j < kJ; ++j)
+                        acc[v][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            as_bf16x8(av[h][i]), as_bf16x8(bv[h][v][j]), acc[v][i][j], 0, 0, 0);
+            if constexpr (kGate) {
+                if (wn == 0u) {  // uniform
+                    const u32x4 zero = {0u, 0u, 0u, 0u};
+                    const u32x4 g = gate_lane ? gv[h] : zero;
+#pragma unroll
+                    for (uint32_t i = 0; i < kI; ++i)
+                        acc_gate[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            as_bf16x8(av[h][i]), as_bf16x8(g), acc_gate[i], 0, 0, 0);
+                }
+            }
+        }
+    };
+    clear();
+    const uint32_t chunks = k / 64u;       // >= kStages - 1
+    const uint32_t quarter = chunks / 4u;  // kSplit
+#pragma unroll
+    for (uint32_t c = 0; c + 1u < kStages; ++c) load(c, c);
+    // step c: chunk c's loads of every wave are done and slot c - 1 is free
+    uint32_t slot = 0u, next_fold = quarter;
+    auto step = [&](uint32_t c) __attribute__((always_inline)) {
+        multiply(c, slot);
+        slot = slot + 1u == kStages ? 0u : slot + 1u;
+        if constexpr (kSplit) {
+            if (c + 1u == next_fold) {
+                fold(next_fold == quarter);
+                next_fold += quarter;
+            }
+        }
+    };
+    uint32_t c = 0;
+    for (; c + kStages - 1u < chunks; ++c) {
+        chunk_barrier<kLoads * (kStages - 2u)>();
+        load(c + kStages - 1u, slot == 0u ? kStages - 1u : slot - 1u);
+        step(c);
+    }
+    // the last kStages - 1 chunks are in flight
+    if constexpr (kStages > 4u) {
+        chunk_barrier<kLoads * 3u>();
+        step(c++);
+    }
+    if constexpr (kStages > 3u) {
+        chunk_barrier<kLoads * 2u>();
+        step(c++);
+    }
+    if constexpr (kStages > 2u) {
+        chunk_barrier<kLoads>();
+        step(c++);
+    }
+    chunk_barrier<0u>();
+    step(c);
+    // D layout: lane l holds rows 4 (l/16) + e of column l%16 of each tile;
+    // finish(row, column, values of the kNB matrices, false) and, with
+    // kGate, finish(row, 0, the gate's value, true); rows and columns may
+    // lie past the matrix
+#pragma unroll
+    for (uint32_t i = 0; i < kI; ++i) {
+#pragma unroll
+        for (uint32_t j = 0; j < kJ; ++j)
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e) {
+                float v[kNB];
+#pragma unroll
+                for (uint32_t x = 0; x < kNB; ++x) {
+                    if constexpr (kSplit) v[x] = total[x][i][j][e];
+                    else v[x] = acc[x][i][j][e];
+                }
+                finish(m0 + a_row + 16u * i + 4u * (lane >> 4) + e,
+                       n0 + 16u * kJ * wn + 16u * j + (lane & 15u), v, false);
+            }
+        if constexpr (kGate) {
+            if (wn == 0u && gate_lane) {
+#pragma unroll
+                for (uint32_t e = 0; e < 4u; ++e) {
+                    float v[kNB] = {total_gate[i][e]};
+                    finish(m0 + a_row + 16u * i + 4u * (lane >> 4) + e, 0u, v, true);
+                }
+            }
+        }
+    }
+}
+
+// Tile of a one-dimensional grid: XCD x (workgroups x, x + 8, ...) runs row
+// tiles x, x + 8, ..., all column tiles of one before the next, so that a row
+// tile's activations are fetched into one L2.
+struct TileAt {
+    uint32_t row, column;
+};
+__device__ __forceinline__ TileAt tile_at(uint32_t column_tiles) {
+    const uint32_t j = blockIdx.x / 8u;
+    return TileAt{j / column_tiles * 8u + blockIdx.x % 8u, j % column_tiles};
+}
+constexpr uint32_t tile_grid(uint32_t row_tiles, uint32_t column_tiles) {
+    return (row_tiles + 7u) / 8u * 8u * column_tiles;
+}
+
+template <typename S, bool kSplit, DenseOut kOut>
+__global__ __launch_bounds__(256, 2) void dense_tile_kernel(
+    const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint32_t m, uint32_t n,
+    uint32_t k, float* __restrict__ c_f32, uint16_t* __restrict__ c_bf16, float divisor,
+    float scale) {
+    __shared__ u32x4 ring[S::kStages * S::kSlot];
+    const TileAt at = tile_at((n + S::kTN - 1u) / S::kTN);
+    const uint32_t m0 = at.row * S::kTM, n0 = at.column * S::kTN;
+    if (m0 >= m) return;
+    tile_product<S, kSplit, false>(
+        a, b, nullptr, m, n, k, m0, n0, ring, nullptr,
+        [&](uint32_t row, uint32_t col, const float (&v)[1], bool) {
+            if (row >= m || col >= n) return;
+            const size_t out = static_cast<size_t>(row) * n + col;
+            if constexpr (kOut == DenseOut::kF32)
+                c_f32[out] = v[0];
+            else
+                c_bf16[out] = static_cast<uint16_t>(dense_epilogue(kOut, v[0], divisor, scale));
+        });
+}
+
+// The shared expert's first half over kTM x (kTN/2) channels per workgroup
+// (see shared_gate_up_kernel); the workgroups of column 0 carry the scalar
+// output gate.
+template <typename S>
+__global__ __launch_bounds__(256, 2) void shared_gate_up_tile_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ w_gate,
+    const uint16_t* __restrict__ w_up, const uint16_t* __restrict__ w_out_gate, uint32_t m,
+    uint32_t inter, uint16_t* __restrict__ g_out, uint16_t* __restrict__ u_out,
+    uint16_t* __restrict__ h_out, uint16_t* __restrict__ gate_out) {
+    __shared__ u32x4 ring[S::kStages * S::kSlot];
+    __shared__ u32x4 gate_lds[kHidden / 8u];
+    static_assert(kHidden / 8u == 256u, "one vector of the gate row per thread");
+    constexpr uint32_t kChannels = S::kTN / 2u;
+    const TileAt at = tile_at((inter + kChannels - 1u) / kChannels);
+    const uint32_t m0 = at.row * S::kTM, n0 = at.column * kChannels;
+    if (m0 >= m) return;
+    auto finish = [&](uint32_t row, uint32_t col, const float (&v)[2], bool gate) {
+        if (row >= m) return;
+        if (gate) {
+            gate_out[row] = static_cast<uint16_t>(f32_to_bf16(v[0]));
+            return;
+        }
+        if (col >= inter) return;
+        const uint32_t g = f32_to_bf16(v[0]), u = f32_to_bf16(v[1]);
+        const size_t out = static_cast<size_t>(row) * inter + col;
+        g_out[out] = static_cast<uint16_t>(g);
+        u_out[out] = static_cast<uint16_t>(u);
+        h_out[out] = static_cast<uint16_t>(silu_multiply(g, u));
+    };
+    if (at.column == 0u) {
+        // stored before the first chunk barrier, which every wave passes
+        gate_lds[threadIdx.x] = reinterpret_cast<const u32x4*>(w_out_gate)[threadIdx.x];
+        tile_product<S, true, true>(x, w_gate, w_up, m, inter, kHidden, m0, n0, ring, gate_lds,
+                                    finish);
+    } else {
+        tile_product<S, true, false>(x, w_gate, w_up, m, inter, kHidden, m0, n0, ring, nullptr,
+                                     finish);
+    }
+}
+
 // ---- one activation row (m = 1: the batch-1 decode step) --------------
 // At m = 1 a GEMM is a GEMV: every weight byte is used once, so the bound is
 // how fast the weight rows stream, and a 16 x 16 MFMA tile would waste 15 of
@@ -638,6 +954,78 @@ namespace {
 // one activation row: the GEMV form (grids of up to 65535 workgroups)
 constexpr uint32_t kGemvMaxRows = 65535u * 4u;
 
+template <typename S, bool kSplit, DenseOut kOut>
+void launch_dense_tile(const uint16_t* a, const uint16_t* b, uint32_t m, uint32_t n, uint32_t k,
+                       float* c_f32, uint16_t* c_bf16, float divisor, float scale,
+                       hipStream_t stream) {
+    dense_tile_kernel<S, kSplit, kOut>
+        <<<tile_grid((m + S::kTM - 1u) / S::kTM, (n + S::kTN - 1u) / S::kTN), 256, 0, stream>>>(
+            a, b, m, n, k, c_f32, c_bf16, divisor, scale);
+}
+
+void launch_shared_small(const uint16_t* hidden, const uint16_t* w_gate, const uint16_t* w_up,
+                         const uint16_t* w_out_gate, uint32_t tokens, uint32_t inter, uint16_t* g,
+                         uint16_t* u, uint16_t* h, uint16_t* gate, hipStream_t stream) {
+    const dim3 grid(inter / 32u, (tokens + 31u) / 32u);
+    shared_gate_up_kernel<<<grid, 256, 0, stream>>>(hidden, w_gate, w_up, w_out_gate, tokens, inter,
+                                                    g, u, h, gate);
+}
+
+template <typename S>
+void launch_shared_tile(const uint16_t* hidden, const uint16_t* w_gate, const uint16_t* w_up,
+                        const uint16_t* w_out_gate, uint32_t tokens, uint32_t inter, uint16_t* g,
+                        uint16_t* u, uint16_t* h, uint16_t* gate, hipStream_t stream) {
+    constexpr uint32_t kChannels = S::kTN / 2u;
+    shared_gate_up_tile_kernel<S>
+        <<<tile_grid((tokens + S::kTM - 1u) / S::kTM, (inter + kChannels - 1u) / kChannels), 256, 0,
+           stream>>>(hidden, w_gate, w_up, w_out_gate, tokens, inter, g, u, h, gate);
+}
+
+// Large products take workgroup tiles: 64 x 64 with three chunks in the ring
+// (three workgroups per CU) from about 200 tiles on, 128 x 128 with two (two
+// per CU) from about 400 of those.  Measured, old kernels / 64 x 64 / 128 x 128,
+// us -- router (512 x 2048): 1,024 rows 9.8 / 11.7 / 24.6, 2,048 rows 16.5 /
+// 12.6 / 24.4, 4,099 rows 31.2 / 19.7 / 25.6, 8,192 rows 54.0 / 31.1 / 28.6,
+// 32,768 rows 226 / 134 / 92.  Shared gate/up: 512 rows 11.1 / 14.9 / 33,
+// 1,024 rows 19.0 / 15.7 / 33, 4,099 rows 73.6 / 32.9 / 36.5, 32,768 rows
+// 531 / 234 / 192.  Shared down (2,048 x 512): 512 rows 5.1 / 4.6 / -, 4,099
+// rows 20.5 / 16.9 / 17.9, 32,768 rows 125 / 136 / 101.
+constexpr uint32_t kTileMinTiles = 192;
+constexpr uint32_t kTile128MinTiles = 384;
+// their one-dimensional grids hold at most 2^32 threads
+constexpr uint64_t kTileMaxTiles = (1ull << 23);
+template <uint32_t kNB>
+using Tile64 = TileShape<64, 64, kNB, 3>;
+template <uint32_t kNB>
+using Tile128 = TileShape<128, 128, kNB, 2>;
+
+// tiles of `rows` rows and `columns` columns over an m x n output
+constexpr uint64_t tile_count(uint32_t m, uint32_t n, uint32_t rows, uint32_t columns) {
+    return (static_cast<uint64_t>(m) + rows - 1u) / rows *
+           ((static_cast<uint64_t>(n) + columns - 1u) / columns);
+}
+
+// the product on workgroup tiles where they are the faster form; kSplit: the
+// summation order of the kernel they stand in for
+template <bool kSplit, DenseOut kOut>
+bool launch_dense_large(const uint16_t* a, const uint16_t* b, uint32_t m, uint32_t n, uint32_t k,
+                        float* c_f32, uint16_t* c_bf16, float divisor, float scale,
+                        hipStream_t stream) {
+    // whole chunks, for the split in every quarter, and as many as a ring's
+    if (k % (kSplit ? 256u : 64u) != 0u || k < 3u * 64u ||
+        tile_count(m, n, 64u, 64u) > kTileMaxTiles)
+        return false;
+    if (tile_count(m, n, 128u, 128u) >= kTile128MinTiles)
+        launch_dense_tile<Tile128<1>, kSplit, kOut>(a, b, m, n, k, c_f32, c_bf16, divisor, scale,
+                                                    stream);
+    else if (tile_count(m, n, 64u, 64u) >= kTileMinTiles)
+        launch_dense_tile<Tile64<1>, kSplit, kOut>(a, b, m, n, k, c_f32, c_bf16, divisor, scale,
+                                                   stream);
+    else
+        return false;
+    return true;
+}
+
 template <DenseOut kOut>
 void launch_dense_tiles(const uint16_t* a, const uint16_t* b, uint32_t m, uint32_t n, uint32_t k,
                         float* c_f32, uint16_t* c_bf16, float divisor, float scale,
@@ -647,15 +1035,23 @@ void launch_dense_tiles(const uint16_t* a, const uint16_t* b, uint32_t m, uint32
                                                              scale);
         return;
     }
-    // short K with a 64 x 64 grid that fills the GPU: workgroup-shared
-    // tiles read half the bytes per output of the K-split 32 x 32 tiles
-    const uint32_t tiles64 = ((m + 63u) / 64u) * ((n + 63u) / 64u);
-    if (k <= kTile64MaxK && tiles64 >= kTile64MinTiles) {
+    // short K with a 64 x 64 grid that fills the GPU: one accumulator over K
+    if (k <= kTile64MaxK && tile_count(m, n, 64u, 64u) >= kTile64MinTiles) {
+        // with an activation (the hyper mix-up, K = 320) the epilogue sets the
+        // time, and the small tiles' is spread wider: 36 us against 40 (64 x
+        // 64 ring) and 46 (128 x 128) for 2,000 x 8,192
+        if constexpr (kOut == DenseOut::kF32 || kOut == DenseOut::kBf16) {
+            if (launch_dense_large<false, kOut>(a, b, m, n, k, c_f32, c_bf16, divisor, scale,
+                                                stream))
+                return;
+        }
         const dim3 grid((n + 63u) / 64u, (m + 63u) / 64u);
         dense_tile64_kernel<kOut><<<grid, 256, 0, stream>>>(a, b, m, n, k, c_f32, c_bf16, divisor,
                                                             scale);
         return;
     }
+    if (launch_dense_large<true, kOut>(a, b, m, n, k, c_f32, c_bf16, divisor, scale, stream))
+        return;
     const uint32_t tm = m <= 16u ? 1u : 2u;
     const uint32_t tn = (m <= 16u || n <= 16u) ? 1u : 2u;
     const dim3 grid((n + 16u * tn - 1u) / (16u * tn), (m + 16u * tm - 1u) / (16u * tm));
@@ -744,9 +1140,16 @@ hipError_t launch_shared_expert(const uint16_t* hidden, const uint16_t* w_gate,
         shared_gate_up_gemv_kernel<<<(inter + 2u) / 2u, 128, 0, stream>>>(
             hidden, w_gate, w_up, w_out_gate, inter, g, u, h, shared_gate);
     } else {
-        const dim3 grid(inter / 32u, (tokens + 31u) / 32u);
-        shared_gate_up_kernel<<<grid, 256, 0, stream>>>(hidden, w_gate, w_up, w_out_gate, tokens,
-                                                        inter, g, u, h, shared_gate);
+        const uint64_t tiles64 = tile_count(tokens, 2u * inter, 64u, 64u);
+        if (tiles64 < kTileMinTiles || tiles64 > kTileMaxTiles)
+            launch_shared_small(hidden, w_gate, w_up, w_out_gate, tokens, inter, g, u, h,
+                                shared_gate, stream);
+        else if (tile_count(tokens, 2u * inter, 128u, 128u) < kTile128MinTiles)
+            launch_shared_tile<Tile64<2>>(hidden, w_gate, w_up, w_out_gate, tokens, inter, g, u, h,
+                                          shared_gate, stream);
+        else
+            launch_shared_tile<Tile128<2>>(hidden, w_gate, w_up, w_out_gate, tokens, inter, g, u,
+                                           h, shared_gate, stream);
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
