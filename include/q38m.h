@@ -492,7 +492,7 @@ int q38m_hyper_mix_bf16(const uint16_t* normalized_hyper, const uint16_t* mix_we
 int q38m_hyper_inject_bf16(const uint16_t* original_hyper, const uint16_t* block_output,
                            const uint16_t* injection_weights, uint16_t* output_hyper,
                            uint32_t tokens, uint32_t hidden, void* stream, int device);
-/* The whole prepare_hyper sequence (cuda_backend.cu:1219-1243) in four
+/* The whole prepare_hyper sequence (cuda_backend.cu:1219-1243) in up to four
  * launches: mix_down [low_rank][4H], mix_up [4H][low_rank], inject [4][4H]
  * or NULL (then injection is not written).  low_rank % 32 == 0.  Outputs
  * mixed [T][H] (the MoE input) and injection [T][4] (for the finish). */

@@ -605,7 +605,8 @@ __global__ __launch_bounds__(256) void shared_gate_up_kernel(
 // The stacked B rows of a tile with kNB = 2 matrices are kTN/2 rows of the
 // first, then the same rows of the second, and a wave's columns are its
 // share of both.  With kGate the waves of column wn = 0 also multiply one
-// extra B row (gate_lds, all of K), as wave_partial does.
+// extra B row (gate_lds, all of K), as wave_partial does.  k columns of rows
+// `pitch` apart.
 template <uint32_t kTM_, uint32_t kTN_, uint32_t kNB_, uint32_t kStages_>
 struct TileShape {
     static constexpr uint32_t kTM = kTM_, kTN = kTN_, kNB = kNB_, kStages = kStages_;
@@ -640,8 +641,9 @@ template <typename S, bool kSplit, bool kGate, typename Finish>
 __device__ __forceinline__ void tile_product(const uint16_t* __restrict__ a,
                                              const uint16_t* __restrict__ b0,
                                              const uint16_t* __restrict__ b1, uint32_t m,
-                                             uint32_t n, uint32_t k, uint32_t m0, uint32_t n0,
-                                             u32x4* ring, const u32x4* gate_lds, Finish finish) {
+                                             uint32_t n, uint32_t pitch, uint32_t k, uint32_t m0,
+                                             uint32_t n0, u32x4* ring, const u32x4* gate_lds,
+                                             Finish finish) {
     constexpr uint32_t kTM = S::kTM, kTN = S::kTN, kNB = S::kNB, kStages = S::kStages;
     constexpr uint32_t kI = S::kI, kJ = S::kJ, kLoads = S::kLoads;
     const uint32_t t = threadIdx.x;
@@ -655,12 +657,12 @@ __device__ __forceinline__ void tile_product(const uint16_t* __restrict__ a,
         const uint32_t row = 32u * i + 8u * wave + (lane >> 3);
         const uint16_t* base;
         if (32u * i < kTM) {
-            base = a + static_cast<size_t>(min(m0 + row, m - 1u)) * k;
+            base = a + static_cast<size_t>(min(m0 + row, m - 1u)) * pitch;
         } else {
             const uint32_t r = row - kTM;
             const bool second = kNB == 2u && 32u * i - kTM >= kTN / 2u;
             base = (second ? b1 : b0) +
-                   static_cast<size_t>(min(n0 + (second ? r - kTN / 2u : r), n - 1u)) * k;
+                   static_cast<size_t>(min(n0 + (second ? r - kTN / 2u : r), n - 1u)) * pitch;
         }
         src[i] = reinterpret_cast<const u32x4*>(base) + ((lane & 7u) ^ ((row >> 1) & 7u));
     }
@@ -845,7 +847,7 @@ __global__ __launch_bounds__(256, 2) void dense_tile_kernel(
     const uint32_t m0 = at.row * S::kTM, n0 = at.column * S::kTN;
     if (m0 >= m) return;
     tile_product<S, kSplit, false>(
-        a, b, nullptr, m, n, k, m0, n0, ring, nullptr,
+        a, b, nullptr, m, n, k, k, m0, n0, ring, nullptr,
         [&](uint32_t row, uint32_t col, const float (&v)[1], bool) {
             if (row >= m || col >= n) return;
             const size_t out = static_cast<size_t>(row) * n + col;
@@ -888,11 +890,206 @@ __global__ __launch_bounds__(256, 2) void shared_gate_up_tile_kernel(
     if (at.column == 0u) {
         // stored before the first chunk barrier, which every wave passes
         gate_lds[threadIdx.x] = reinterpret_cast<const u32x4*>(w_out_gate)[threadIdx.x];
-        tile_product<S, true, true>(x, w_gate, w_up, m, inter, kHidden, m0, n0, ring, gate_lds,
-                                    finish);
+        tile_product<S, true, true>(x, w_gate, w_up, m, inter, kHidden, kHidden, m0, n0, ring,
+                                    gate_lds, finish);
     } else {
-        tile_product<S, true, false>(x, w_gate, w_up, m, inter, kHidden, m0, n0, ring, nullptr,
-                                     finish);
+        tile_product<S, true, false>(x, w_gate, w_up, m, inter, kHidden, kHidden, m0, n0, ring,
+                                     nullptr, finish);
+    }
+}
+
+// ---- hyper-connection low-rank products on workgroup tiles -----------------
+
+// One K quarter of C = A * B^T on 64 x 64 tiles, quarter q = blockIdx.y:
+// fp32 partials [q][m][n].  A low-rank projection over K = 4H has few tiles
+// (160 at 2,000 tokens and rank 320), so its quarters run side by side: 47.9 us
+// on 32 x 32 tiles -> 21.3 us, and 4.8 us for the sum.
+template <typename S>
+__global__ __launch_bounds__(256, 2) void dense_quarter_kernel(const uint16_t* __restrict__ a,
+                                                               const uint16_t* __restrict__ b,
+                                                               uint32_t m, uint32_t n, uint32_t k,
+                                                               float* __restrict__ partials) {
+    __shared__ u32x4 ring[S::kStages * S::kSlot];
+    const TileAt at = tile_at((n + S::kTN - 1u) / S::kTN);
+    const uint32_t m0 = at.row * S::kTM, n0 = at.column * S::kTN;
+    if (m0 >= m) return;
+    const uint32_t q = blockIdx.y, span = k / 4u;
+    float* out = partials + static_cast<size_t>(q) * m * n;
+    tile_product<S, false, false>(
+        a + static_cast<size_t>(q) * span, b + static_cast<size_t>(q) * span, nullptr, m, n, k,
+        span, m0, n0, ring, nullptr,
+        [&](uint32_t row, uint32_t col, const float (&v)[1], bool) {
+            if (row < m && col < n) out[static_cast<size_t>(row) * n + col] = v[0];
+        });
+}
+
+// The quarters' partials summed in order (the sums of dense_gemm_kernel's
+// four waves), then the SiLU step; 4 values a thread.
+__global__ __launch_bounds__(256) void quarter_silu_kernel(const f32x4* __restrict__ partials,
+                                                           uint32_t total4, float divisor,
+                                                           uint16_t* __restrict__ out) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= total4) return;
+    f32x4 sum = partials[i];
+#pragma unroll
+    for (uint32_t q = 1; q < 4u; ++q) sum += partials[static_cast<size_t>(q) * total4 + i];
+    uint32_t w[4];
+#pragma unroll
+    for (uint32_t e = 0; e < 4u; ++e)
+        w[e] = dense_epilogue(DenseOut::kBf16Silu, sum[e], divisor, 1.0f);
+    reinterpret_cast<uint2*>(out)[i] = make_uint2(w[0] | (w[1] << 16), w[2] | (w[3] << 16));
+}
+
+// The mix-up product, its sigmoid and the stream mix in one kernel
+// (q38_hyper.cu:87-114 over the GEMM of cuda_backend.cu:1228-1236): the
+// [T][4H] mix weights never reach memory.  A workgroup covers 128 tokens x 32
+// channels of all four streams, each wave 32 of the tokens: mix_up's rows
+// are the MFMA's A operand, so a lane holds channels of one token.  LDS row
+// 32 s + 16 i + r of a chunk (stream s, tile i, row r) keeps channel
+// 8 (r/4) + 4 i + r%4, which leaves lane (q, n) channels 8q .. 8q + 7 of
+// token n: one 16-byte piece per stream of `normalized` and of `mixed`.  K
+// (the rank) runs in whole or, at its end, half 64-wide chunks through the
+// ring of tile_product, one accumulator over all of K; a half chunk's loads
+// repeat its first half.  The values are those of the product, the sigmoid
+// and the mix as separate launches, bit for bit.
+//
+// What bounds it: the delivery of mix_up's and low's rows (164 KB per workgroup
+// at rank 320 and 128 tokens) and the VALU's share of 16.4 M sigmoids at 2,000
+// tokens.  The sigmoid's argument and result are bf16, so it is read from a
+// table in LDS (kSigmoidTable, 4,096 fp32 words; ~8 VALU instructions instead
+// of ~50 with the exp and the division; NaN passes through).
+__device__ const uint32_t kSigmoidTable[4096] = {
+#include "q38m_sigmoid_table.inc"
+};
+
+__global__ __launch_bounds__(256, 2) void hyper_mix_up_kernel(
+    const uint16_t* __restrict__ low, const uint16_t* __restrict__ up,
+    const uint16_t* __restrict__ normalized, uint32_t tokens, uint32_t hidden, uint32_t rank,
+    uint16_t* __restrict__ mixed) {
+    constexpr uint32_t kStreams = 4, kTokens = 128, kChannels = 32, kStages = 2;
+    constexpr uint32_t kJ = kTokens / 64u;  // a wave's token tiles
+    constexpr uint32_t kRows = kStreams * kChannels + kTokens;
+    constexpr uint32_t kSlot = kRows * 8u, kLoads = kRows / 32u;
+    __shared__ u32x4 ring[kStages * kSlot];
+    __shared__ u32x4 sigmoid_lds[1024];
+    // by pairs of column tiles (the halves of 128-byte lines): an XCD runs
+    // every token tile of a pair before the next pair, so that mix_up's rows
+    // are fetched into one L2
+    const TileAt at = tile_at(2u * ((tokens + kTokens - 1u) / kTokens));
+    const uint32_t t0 = at.column / 2u * kTokens;
+    const uint32_t c0 = (2u * at.row + at.column % 2u) * kChannels;
+    if (c0 >= hidden) return;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t n = lane & 15u, q = lane >> 4;
+
+    // load i of the wave: LDS rows 8 (4 i + wave) + lane/8, position lane%8
+    const u32x4* src[kLoads];
+    const uint32_t chunk = (lane & 7u) ^ ((4u * wave + (lane >> 4)) & 7u);
+#pragma unroll
+    for (uint32_t i = 0; i < kLoads; ++i) {
+        const uint32_t row = 32u * i + 8u * wave + (lane >> 3);
+        const uint16_t* base;
+        if (32u * i < kStreams * kChannels) {
+            const uint32_t r = row & 15u, tile = (row >> 4) & 1u;
+            const uint32_t channel = c0 + 8u * (r >> 2) + 4u * tile + (r & 3u);
+            base = up + (static_cast<size_t>(i) * hidden + channel) * rank;
+        } else {
+            base = low + static_cast<size_t>(min(t0 + row - kStreams * kChannels, tokens - 1u)) * rank;
+        }
+        src[i] = reinterpret_cast<const u32x4*>(base) + chunk;
+    }
+    const uint32_t steps = rank / 32u, chunks = (steps + 1u) / 2u;
+    const uint32_t back = chunk < 4u ? 0u : 4u;
+    auto load = [&](uint32_t c, uint32_t slot) __attribute__((always_inline)) {
+        const uint32_t shift = 2u * c + 1u < steps ? 0u : back;
+#pragma unroll
+        for (uint32_t i = 0; i < kLoads; ++i)
+            load_to_lds(src[i] + 8u * c - shift, ring + slot * kSlot + (4u * i + wave) * 64u);
+    };
+    load(0u, 0u);
+    // stored before the first chunk barrier, which every wave passes
+    const u32x4* table = reinterpret_cast<const u32x4*>(kSigmoidTable);
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; ++i) sigmoid_lds[256u * i + threadIdx.x] = table[256u * i + threadIdx.x];
+    // the normalized pieces arrive while the product runs
+    u32x4 norm[kJ][kStreams];
+#pragma unroll
+    for (uint32_t j = 0; j < kJ; ++j) {
+        const uint32_t token = min(t0 + 16u * kJ * wave + 16u * j + n, tokens - 1u);
+#pragma unroll
+        for (uint32_t s = 0; s < kStreams; ++s)
+            norm[j][s] = *reinterpret_cast<const u32x4*>(
+                normalized + (static_cast<size_t>(token) * kStreams + s) * hidden + c0 + 8u * q);
+    }
+    const uint32_t swizzle = (lane >> 1) & 7u;
+    const uint32_t read_slot[2] = {8u * n + (q ^ swizzle), 8u * n + ((4u + q) ^ swizzle)};
+    const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 acc[kStreams][2][kJ];  // [stream][channel tile][token tile]
+#pragma unroll
+    for (uint32_t s = 0; s < kStreams; ++s)
+#pragma unroll
+        for (uint32_t i = 0; i < 2u; ++i)
+#pragma unroll
+            for (uint32_t j = 0; j < kJ; ++j) acc[s][i][j] = zero4;
+    for (uint32_t c = 0; c < chunks; ++c) {
+        // chunk c has landed everywhere and its predecessor's slot is free
+        chunk_barrier<0u>();
+        if (c + 1u < chunks) load(c + 1u, (c + 1u) & 1u);
+        const u32x4* lds = ring + (c & 1u) * kSlot;
+#pragma unroll
+        for (uint32_t h = 0; h < 2u; ++h) {
+            if (2u * c + h >= steps) break;
+            u32x4 av[kStreams][2], bv[kJ];
+#pragma unroll
+            for (uint32_t j = 0; j < kJ; ++j)
+                bv[j] = lds[8u * (kStreams * kChannels + 16u * kJ * wave + 16u * j) + read_slot[h]];
+#pragma unroll
+            for (uint32_t s = 0; s < kStreams; ++s)
+#pragma unroll
+                for (uint32_t i = 0; i < 2u; ++i)
+                    av[s][i] = lds[8u * (32u * s + 16u * i) + read_slot[h]];
+#pragma unroll
+            for (uint32_t s = 0; s < kStreams; ++s)
+#pragma unroll
+                for (uint32_t i = 0; i < 2u; ++i)
+#pragma unroll
+                    for (uint32_t j = 0; j < kJ; ++j)
+                        acc[s][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            as_bf16x8(av[s][i]), as_bf16x8(bv[j]), acc[s][i][j], 0, 0, 0);
+        }
+    }
+    const float* sigmoid_table = reinterpret_cast<const float*>(sigmoid_lds);
+    auto sigmoid = [&](uint32_t word) __attribute__((always_inline)) {
+        const uint32_t magnitude = word & 0x7fffu;
+        const uint32_t at = min(max(magnitude, 0x3b00u), 0x42ffu) - 0x3b00u + ((word >> 4) & 0x800u);
+        const float value = sigmoid_table[at];
+        return magnitude > 0x7f80u ? bf16_to_f32(word) : value;
+    };
+#pragma unroll
+    for (uint32_t j = 0; j < kJ; ++j) {
+        const uint32_t token = t0 + 16u * kJ * wave + 16u * j + n;
+        uint32_t w[4];
+#pragma unroll
+        for (uint32_t v = 0; v < 4u; ++v) {
+            uint32_t word[2];
+#pragma unroll
+            for (uint32_t b = 0; b < 2u; ++b) {
+                const uint32_t e = 2u * v + b;  // channel c0 + 8q + e: tile e/4, element e%4
+                float sum = 0.0f;
+#pragma unroll
+                for (uint32_t s = 0; s < kStreams; ++s) {
+                    const float mix = sigmoid(f32_to_bf16(acc[s][e >> 2][j][e & 3u]));
+                    const uint32_t pair = norm[j][s][v];
+                    sum = __builtin_fmaf(bf16_to_f32(b ? pair >> 16 : pair & 0xffffu), mix, sum);
+                }
+                word[b] = f32_to_bf16(sum / static_cast<float>(kStreams));
+            }
+            w[v] = word[0] | (word[1] << 16);
+        }
+        if (token < tokens)
+            *reinterpret_cast<uint4*>(mixed + static_cast<size_t>(token) * hidden + c0 + 8u * q) =
+                make_uint4(w[0], w[1], w[2], w[3]);
     }
 }
 
@@ -1087,6 +1284,46 @@ hipError_t launch_dense_gemm_act(const uint16_t* a, const uint16_t* b, uint32_t 
         launch_dense_tiles<DenseOut::kBf16Sigmoid>(a, b, m, n, k, nullptr, c_bf16, divisor,
                                                    scale, stream);
     return hipGetLastError();
+}
+
+// Above this many tokens the prepare's products run on workgroup tiles (a
+// prepare of up to 512 tokens leaves its stages in the scratch).
+constexpr uint32_t kHyperTileMinTokens = 513;
+
+bool launch_hyper_mix_down(const uint16_t* x, const uint16_t* mix_down, uint32_t tokens,
+                           uint32_t rank, uint32_t width, float divisor, float* partials,
+                           uint16_t* low, hipStream_t stream, hipError_t* status) {
+    using S = Tile64<1>;
+    const uint64_t tiles = tile_count(tokens, rank, 64u, 64u);
+    // two whole tiles per CU and more keep K in one workgroup (no second
+    // launch); the quarters must be whole chunks
+    if (tokens < kHyperTileMinTokens || tiles >= 512u || width % 256u != 0u ||
+        width / 256u < S::kStages || (static_cast<uint64_t>(tokens) * rank) % 4u != 0u)
+        return false;
+    dense_quarter_kernel<S>
+        <<<dim3(tile_grid((tokens + 63u) / 64u, (rank + 63u) / 64u), 4), 256, 0, stream>>>(
+            x, mix_down, tokens, rank, width, partials);
+    const uint32_t total4 = tokens * rank / 4u;
+    quarter_silu_kernel<<<(total4 + 255u) / 256u, 256, 0, stream>>>(
+        reinterpret_cast<const f32x4*>(partials), total4, divisor, low);
+    *status = hipGetLastError();
+    return true;
+}
+
+bool launch_hyper_mix_up(const uint16_t* low, const uint16_t* mix_up, const uint16_t* normalized,
+                         uint32_t tokens, uint32_t hidden, uint32_t rank, uint16_t* mixed,
+                         hipStream_t stream, hipError_t* status) {
+    const uint64_t workgroups = (static_cast<uint64_t>(tokens) + 127u) / 128u * (hidden / 32u);
+    // the shapes whose product runs over one accumulator (launch_dense_tiles)
+    if (tokens < kHyperTileMinTokens || hidden % 32u != 0u || rank % 32u != 0u ||
+        rank > kTile64MaxK || tile_count(tokens, 4u * hidden, 64u, 64u) < kTile64MinTiles ||
+        workgroups > kTileMaxTiles)
+        return false;
+    hyper_mix_up_kernel<<<tile_grid((hidden + 63u) / 64u, 2u * ((tokens + 127u) / 128u)), 256, 0,
+                          stream>>>(
+        low, mix_up, normalized, tokens, hidden, rank, mixed);
+    *status = hipGetLastError();
+    return true;
 }
 
 size_t router_topk_workspace_bytes(uint32_t tokens) {

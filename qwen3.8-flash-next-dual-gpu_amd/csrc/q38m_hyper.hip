@@ -300,12 +300,20 @@ hipError_t launch_hyper_prepare(const uint16_t* hyper, const uint16_t* norm_weig
     uint16_t* low = mix + static_cast<size_t>(tokens) * width;
     hipError_t e = launch_hyper_norm(hyper, norm_weight, inject, tokens, hidden, normalized,
                                      injection, stream);
-    if (e == hipSuccess)
+    if (e != hipSuccess) return e;
+    // the mix region holds the mix-down's fp32 partials until the mix weights
+    // are written (16 rank bytes per token against 8 hidden)
+    const bool partials_fit = 2u * low_rank <= hidden;
+    if (!(partials_fit &&
+          launch_hyper_mix_down(normalized, mix_down, tokens, low_rank, width,
+                                static_cast<float>(kStreams), reinterpret_cast<float*>(mix), low,
+                                stream, &e)))
         e = launch_dense_gemm_act(normalized, mix_down, tokens, low_rank, width, true,
                                   static_cast<float>(kStreams), 1.0f, low, stream);
-    if (e == hipSuccess)
-        e = launch_dense_gemm_act(low, mix_up, tokens, width, low_rank, false, 1.0f, 1.0f, mix,
-                                  stream);
+    if (e != hipSuccess) return e;
+    if (launch_hyper_mix_up(low, mix_up, normalized, tokens, hidden, low_rank, mixed, stream, &e))
+        return e;
+    e = launch_dense_gemm_act(low, mix_up, tokens, width, low_rank, false, 1.0f, 1.0f, mix, stream);
     if (e == hipSuccess) e = launch_hyper_mix(normalized, mix, mixed, tokens, hidden, stream);
     return e;
 }

@@ -172,6 +172,18 @@ hipError_t launch_dense_gemm(const uint16_t* a, const uint16_t* b, uint32_t m, u
 hipError_t launch_dense_gemm_act(const uint16_t* a, const uint16_t* b, uint32_t m, uint32_t n,
                                  uint32_t k, bool silu, float divisor, float scale,
                                  uint16_t* c_bf16, hipStream_t stream);
+// the hyper-connection prepare's low-rank products on workgroup tiles; each
+// returns false, having launched nothing, where its tiles do not fit the
+// shape or are not the faster form (status: the launches' result).
+// low = bf16(silu(bf16(x * mix_down^T) / divisor)) through fp32 partials
+// [4][tokens][rank] of the four K quarters
+bool launch_hyper_mix_down(const uint16_t* x, const uint16_t* mix_down, uint32_t tokens,
+                           uint32_t rank, uint32_t width, float divisor, float* partials,
+                           uint16_t* low, hipStream_t stream, hipError_t* status);
+// mixed = the stream mix of `normalized` with sigmoid(bf16(low * mix_up^T))
+bool launch_hyper_mix_up(const uint16_t* low, const uint16_t* mix_up, const uint16_t* normalized,
+                         uint32_t tokens, uint32_t hidden, uint32_t rank, uint16_t* mixed,
+                         hipStream_t stream, hipError_t* status);
 // router logits with the top-10 selection: level 1 in the GEMM epilogue,
 // level 2 in a second launch; the workspace holds the candidate keys
 size_t router_topk_workspace_bytes(uint32_t tokens);

@@ -1,5 +1,6 @@
-/* Build-time generator of the SwiGLU gate table used by the chunk-path
- * gate/up kernels (csrc/q38m_wide.hip).
+/* Build-time generator of two activation tables: the SwiGLU gate of the
+ * chunk-path gate/up kernels (csrc/q38m_wide.hip) and the stream-mix sigmoid
+ * of the hyper-connection prepare (csrc/q38m_dense.hip).
  *
  * The gate value enters SwiGLU already rounded to bf16
  * (cuda/q38_moe_prefill.cu:449-461: g = bf16(y_gate), silu = g/(1+exp(-g))),
@@ -15,7 +16,14 @@
  * for the same g (the tests compare all 65,536 entries with the oracle,
  * NaN results as NaN).
  *
+ * The sigmoid's argument and result are bf16 too (q38_hyper.cu:87-97), and
+ * outside 2^-9 <= |v| < 2^7 the result is that of the nearer end (0.5, or 0
+ * and 1), so `sigmoid` prints only those magnitudes: entry 2048 s + i holds
+ * the fp32 word of bf16(1 / (1 + exp(-v))), v the bf16 with sign s and
+ * magnitude word 0x3b00 + i.
+ *
  * Usage: q38m_silu_gen > q38m_silu_table.inc
+ *        q38m_silu_gen sigmoid > q38m_sigmoid_table.inc
  */
 #include <math.h>
 #include <stdint.h>
@@ -57,7 +65,25 @@ static float exp_contract(float x) {
     return x != x ? x + x : ranged;
 }
 
-int main(void) {
+/* round to nearest even, finite v */
+static uint32_t bf16_word(float v) {
+    const uint32_t b = to_bits(v);
+    return (b + 0x7fffu + ((b >> 16) & 1u)) >> 16;
+}
+
+static int print_sigmoid(void) {
+    printf("/* bf16(1 / (1 + exp(-v))) as fp32 words, entry 2048 s + i: v = bf16 word\n"
+           " * s << 15 | (0x3b00 + i); written by q38m_silu_gen. */\n");
+    for (uint32_t h = 0; h < 4096u; ++h) {
+        const float v = from_bits(((h >> 11) << 31) | ((0x3b00u + (h & 2047u)) << 16));
+        const float sigmoid = 1.0f / (1.0f + exp_contract(-v));
+        printf("0x%08xu,%c", bf16_word(sigmoid) << 16, (h % 8u) == 7u ? '\n' : ' ');
+    }
+    return ferror(stdout) ? 1 : 0;
+}
+
+int main(int argc, char** argv) {
+    if (argc > 1) return strcmp(argv[1], "sigmoid") == 0 ? print_sigmoid() : 2;
     printf("/* silu(g) = g / (1 + exp(-g)) for every bf16 g (entry h: g = bits h << 16),\n"
            " * fp32 result words; written by q38m_silu_gen. */\n");
     for (uint32_t h = 0; h < 65536u; ++h) {
