@@ -707,8 +707,12 @@ int q38m_moe_prefill_wide_v1(const q38m_expert_weights_v1* gate_up,
     else
         status = q38m::launch_quantize_rows(hidden, tokens, Q38M_HIDDEN, ws->xq, ws->xs, s);
     if (status == hipSuccess)
-        status = q38m::launch_build_wide_plan(ws->expert_ids, tokens, ws->plan,
-                                              wide->plan_scratch, s);
+        // the chunk counts pass through the quantised mid rows, all of which
+        // the mid quantiser writes later: plan_scratch holds the counts of
+        // 2048-route chunks only (513 words per started 512 routes fit 128
+        // words per route from 5 routes on)
+        status = q38m::launch_step_wide_plan(ws->expert_ids, tokens, ws->plan,
+                                             reinterpret_cast<uint32_t*>(ws->mid_q), s);
     if (status == hipSuccess)
         status = q38m::launch_gate_up_wide(*gate_up, ws->xq, ws->xs, ws->plan.packed_assignment,
                                            ws->expert_weights, ws->plan.tasks, tasks,

@@ -58,6 +58,11 @@ uint32_t wide_chunks(uint32_t tokens);
 hipError_t launch_build_wide_plan(const int32_t* ids, uint32_t tokens,
                                   const q38m_route_plan_v1& plan, uint32_t* chunk_counts,
                                   hipStream_t stream);
+// the same plan through shorter chunks where there are few routes;
+// chunk_counts: ceil(routes / 512) * 513 uint32
+hipError_t launch_step_wide_plan(const int32_t* ids, uint32_t tokens,
+                                 const q38m_route_plan_v1& plan, uint32_t* chunk_counts,
+                                 hipStream_t stream);
 // the grouped GEMMs over 128-row tasks, for the formats launch_gate_up /
 // launch_down take; task_count is the number of task slots (zero records
 // past the plan's tasks)

@@ -44,14 +44,15 @@ __device__ const uint32_t kSiluTable[65536] = {
 
 // ---- plan -------------------------------------------------------------------
 
+template <uint32_t kChunkRoutes>
 __global__ __launch_bounds__(256) void wide_count_kernel(const int32_t* __restrict__ ids,
                                                          uint32_t routes,
                                                          uint32_t* __restrict__ chunk_counts) {
     __shared__ uint32_t hist[kCountSlots];
     for (uint32_t i = threadIdx.x; i < kCountSlots; i += 256u) hist[i] = 0u;
     __syncthreads();
-    const uint32_t begin = blockIdx.x * kWideChunkRoutes;
-    const uint32_t end = min(begin + kWideChunkRoutes, routes);
+    const uint32_t begin = blockIdx.x * kChunkRoutes;
+    const uint32_t end = min(begin + kChunkRoutes, routes);
     for (uint32_t a = begin + threadIdx.x; a < end; a += 256u) {
         const int32_t id = ids[a];
         const bool valid = id >= 0 && id < static_cast<int32_t>(kExperts);
@@ -230,6 +231,7 @@ __global__ __launch_bounds__(512) void wide_scan_kernel(uint32_t* __restrict__ c
 // lane ORs its bit into its id's slot, reads the slot back, clears it; one
 // wave's LDS operations execute in order); the stable position is the
 // chunk's running base for the id plus the equal lanes below.
+template <uint32_t kChunkRoutes>
 __global__ __launch_bounds__(64) void wide_scatter_kernel(const int32_t* __restrict__ ids,
                                                           uint32_t routes,
                                                           const uint32_t* __restrict__ bases,
@@ -238,12 +240,12 @@ __global__ __launch_bounds__(64) void wide_scatter_kernel(const int32_t* __restr
     __shared__ unsigned long long table[kCountSlots];
     const uint32_t lane = threadIdx.x;
     const uint32_t* base = bases + static_cast<size_t>(blockIdx.x) * kCountSlots;
-    const uint32_t begin = blockIdx.x * kWideChunkRoutes;
-    const uint32_t end = min(begin + kWideChunkRoutes, routes);
+    const uint32_t begin = blockIdx.x * kChunkRoutes;
+    const uint32_t end = min(begin + kChunkRoutes, routes);
     // every load of the chunk is issued before the first use: the segment
     // bases and the chunk's ids (clamped to its last route, unused past it)
-    constexpr uint32_t kPerLane = kExperts / 64u, kSteps = kWideChunkRoutes / 64u;
-    static_assert(kExperts % 64u == 0u && kWideChunkRoutes % 64u == 0u, "whole waves");
+    constexpr uint32_t kPerLane = kExperts / 64u, kSteps = kChunkRoutes / 64u;
+    static_assert(kExperts % 64u == 0u && kChunkRoutes % 64u == 0u, "whole waves");
     uint32_t offset[kPerLane], chunk_base[kPerLane];
     int32_t idv[kSteps];
 #pragma unroll
@@ -1329,16 +1331,47 @@ uint32_t wide_chunks(uint32_t tokens) {
     return (routes_v1(tokens) + kWideChunkRoutes - 1u) / kWideChunkRoutes;
 }
 
+namespace {
+
+template <uint32_t kChunkRoutes>
+hipError_t build_wide_plan(const int32_t* ids, uint32_t tokens, const q38m_route_plan_v1& plan,
+                           uint32_t* chunk_counts, hipStream_t stream) {
+    const uint32_t routes = routes_v1(tokens);
+    const uint32_t chunks = (routes + kChunkRoutes - 1u) / kChunkRoutes;
+    wide_count_kernel<kChunkRoutes><<<chunks, 256, 0, stream>>>(ids, routes, chunk_counts);
+    wide_scan_kernel<<<1, 512, 0, stream>>>(chunk_counts, chunks, tokens, plan,
+                                            max_tasks_wide(tokens));
+    wide_scatter_kernel<kChunkRoutes><<<chunks, 64, 0, stream>>>(ids, routes, chunk_counts, plan);
+    return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_build_wide_plan(const int32_t* ids, uint32_t tokens,
                                   const q38m_route_plan_v1& plan, uint32_t* chunk_counts,
                                   hipStream_t stream) {
+    return build_wide_plan<kWideChunkRoutes>(ids, tokens, plan, chunk_counts, stream);
+}
+
+// The step's plan cuts the routes into shorter chunks where there are few of
+// them.  The scatter kernel walks a chunk in serial rounds of 64 routes, so
+// its time is the chunk's length (2048 routes: 9.2 us at any token count,
+// 1024: 5.8-6.4, 512: 3.6); the scan reads two batches of 32 chunk counts at
+// once and takes a round trip more for each further batch (15 us at 160
+// chunks), hence the shortest chunk that leaves at most 64.  Step with
+// 2048-route chunks -> this rule: 600 tokens 240.5 -> 234.4 us, 1,500 tokens
+// W8 g128 343.0 -> 338.5 us, 4,096 tokens W4/W8 512.0 -> 507.6 us; 6,001
+// tokens within the runs' difference.
+hipError_t launch_step_wide_plan(const int32_t* ids, uint32_t tokens,
+                                 const q38m_route_plan_v1& plan, uint32_t* chunk_counts,
+                                 hipStream_t stream) {
+    constexpr uint32_t kChunks = 64;
     const uint32_t routes = routes_v1(tokens);
-    const uint32_t chunks = wide_chunks(tokens);
-    wide_count_kernel<<<chunks, 256, 0, stream>>>(ids, routes, chunk_counts);
-    wide_scan_kernel<<<1, 512, 0, stream>>>(chunk_counts, chunks, tokens, plan,
-                                            max_tasks_wide(tokens));
-    wide_scatter_kernel<<<chunks, 64, 0, stream>>>(ids, routes, chunk_counts, plan);
-    return hipGetLastError();
+    if (routes <= kChunks * 512u)
+        return build_wide_plan<512>(ids, tokens, plan, chunk_counts, stream);
+    if (routes <= kChunks * 1024u)
+        return build_wide_plan<1024>(ids, tokens, plan, chunk_counts, stream);
+    return build_wide_plan<2048>(ids, tokens, plan, chunk_counts, stream);
 }
 
 namespace {
