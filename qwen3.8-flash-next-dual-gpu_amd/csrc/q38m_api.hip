@@ -191,9 +191,8 @@ int q38m_topk_router_f32(const float* logits, int32_t* expert_ids, float* expert
         return fail(Q38M_ERR_INVALID_ARGUMENT, "invalid top-k router buffers");
     if (int rc = select_device(device)) return rc;
     if (experts == Q38M_ROUTE_EXPERTS && top_k <= Q38M_ROUTE_TOPK && normalize_top_k)
-        return finish(q38m::launch_route_quantize(logits, nullptr, tokens, top_k, expert_ids,
-                                                  expert_weights, nullptr, nullptr,
-                                                  as_stream(stream)),
+        return finish(q38m::launch_route(logits, tokens, top_k, expert_ids, expert_weights,
+                                         as_stream(stream)),
                       "route_quantize_kernel");
     return finish(q38m::launch_topk(logits, expert_ids, expert_weights, tokens, experts, top_k,
                                     normalize_top_k, as_stream(stream)),

@@ -86,7 +86,10 @@ hipError_t launch_topk(const uint16_t* logits, int32_t* ids, float* weights,
 hipError_t launch_route_quantize_wave(const float* logits, const uint16_t* hidden,
                                      uint32_t tokens, int32_t* ids, float* weights, int8_t* xq,
                                      float* xs, hipStream_t stream);
-// 512 bf16 logits per token, top_k <= 10, normalised (ranked-key kernel)
+// 512 fp32 logits per token, top_k <= 10, normalised
+hipError_t launch_route(const float* logits, uint32_t tokens, uint32_t top_k, int32_t* ids,
+                        float* weights, hipStream_t stream);
+// the same for bf16 logits (ranked-key kernel)
 hipError_t launch_route_bf16(const uint16_t* logits, uint32_t tokens, uint32_t top_k,
                              int32_t* ids, float* weights, hipStream_t stream);
 // 512 experts, top_k <= 10, normalised; hidden may be null (top-k only)

@@ -118,8 +118,10 @@ __global__ __launch_bounds__(256) void topk_kernel(
 // tokens in flight per CU where the ten-wave workgroups of
 // route_quantize_kernel keep three.  (Ten rounds of a wave-wide argmax, each
 // six shuffle steps through the LDS crossbar, took 88 us per 32,768-token
-// layer, VALU-bound.)
+// layer, VALU-bound.)  Without kQuantize, the top-k alone (hidden, xq and xs
+// unused).
 // ---------------------------------------------------------------------------
+template <bool kQuantize>
 __global__ __launch_bounds__(256) void route_quantize_wave_kernel(
     const float* __restrict__ logits, const uint16_t* __restrict__ hidden, uint32_t tokens,
     int32_t* __restrict__ ids, float* __restrict__ weights, int8_t* __restrict__ xq,
@@ -138,8 +140,10 @@ __global__ __launch_bounds__(256) void route_quantize_wave_kernel(
 #pragma unroll
     for (uint32_t j = 0; j < kPerLane; ++j) v[j] = row[lane + 64u * j];
     uint4 h[kChunks];
+    if constexpr (kQuantize) {
 #pragma unroll
-    for (uint32_t c = 0; c < kChunks; ++c) h[c] = src[c * 64u + lane];
+        for (uint32_t c = 0; c < kChunks; ++c) h[c] = src[c * 64u + lane];
+    }
 
     int32_t my_id = 0;
     uint32_t my_rank = 0u;
@@ -158,6 +162,7 @@ __global__ __launch_bounds__(256) void route_quantize_wave_kernel(
         ids[static_cast<size_t>(token) * kTopK + my_rank] = my_id;
         weights[static_cast<size_t>(token) * kTopK + my_rank] = numerator / denominator;
     }
+    if constexpr (!kQuantize) return;
 
     float amax = 0.0f;
 #pragma unroll
@@ -634,8 +639,22 @@ hipError_t launch_route_quantize(const float* logits, const uint16_t* hidden, ui
 hipError_t launch_route_quantize_wave(const float* logits, const uint16_t* hidden,
                                      uint32_t tokens, int32_t* ids, float* weights, int8_t* xq,
                                      float* xs, hipStream_t stream) {
-    route_quantize_wave_kernel<<<(tokens + 3u) / 4u, 256, 0, stream>>>(logits, hidden, tokens,
-                                                                      ids, weights, xq, xs);
+    route_quantize_wave_kernel<true><<<(tokens + 3u) / 4u, 256, 0, stream>>>(
+        logits, hidden, tokens, ids, weights, xq, xs);
+    return hipGetLastError();
+}
+
+// One wave per token from 1,280 tokens on; below, a token's ten waves finish
+// sooner.  Workgroup / wave per token, us: 512 tokens 4.2 / 5.2, 1,024 5.0 /
+// 5.7, 1,500 6.4 / 5.7, 4,099 14.0 / 7.6, 32,768 101.9 / 28.3.
+hipError_t launch_route(const float* logits, uint32_t tokens, uint32_t top_k, int32_t* ids,
+                        float* weights, hipStream_t stream) {
+    constexpr uint32_t kWaveTokens = 1280;
+    if (top_k != kTopK || tokens < kWaveTokens)
+        return launch_route_quantize(logits, nullptr, tokens, top_k, ids, weights, nullptr,
+                                     nullptr, stream);
+    route_quantize_wave_kernel<false><<<(tokens + 3u) / 4u, 256, 0, stream>>>(
+        logits, nullptr, tokens, ids, weights, nullptr, nullptr);
     return hipGetLastError();
 }
 
