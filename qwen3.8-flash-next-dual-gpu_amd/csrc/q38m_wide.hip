@@ -295,31 +295,56 @@ __global__ __launch_bounds__(64) void wide_scatter_kernel(const int32_t* __restr
 // The grouped GEMMs below run on one-dimensional grids of (task, slice)
 // pairs, `slices` slices of the output channels per task slot.  The
 // dispatcher hands workgroups to the 8 XCDs round-robin by id, and each XCD
-// has its own L2: XCD x gets the blocks of kTaskBlock consecutive tasks x,
-// x + 8, x + 16, ..., a task's slices next to each other, so that the slices
-// read the same rows, and an expert's neighbouring tasks the same weights,
-// from one L2.  Small blocks keep the XCDs' loads alike (contiguous eighths
-// of the tasks differ by 10-30 % in rows for 1,500 to 6,000 tokens), and the
-// map needs no word of the plan, so a workgroup's first read is its task
-// record; slots past the plan's tasks hold zero records.
+// has its own L2; a task's slices next to each other on one XCD read the
+// same rows, and an expert's neighbouring tasks the same weights, from one
+// L2.  Two maps:
+// - up to kBlockedSlots task slots and in every wide_i8_kernel, XCD x gets the blocks of kTaskBlock
+//   consecutive tasks x, x + 8, x + 16, ...: the XCDs' loads are alike
+//   (contiguous eighths of the tasks differ by 10-30 % in rows for 1,500 to
+//   6,000 tokens), and the map needs no word of the plan, so a workgroup's
+//   first read is its task record; slots past the plan's tasks hold zero
+//   records.
+// - above, the kernels of groups of 32 and of W8 per-channel down give each
+//   XCD a contiguous eighth of the plan's tasks: the eighths are alike by
+//   then, and a hot expert's tasks stay in one L2.  32,768 tokens W4/W8, Zipf
+//   0.8: 3,073 us against 3,112 with blocks of four (16,384 tokens: 1,685
+//   against 1,678).  The 32x32 kernels keep the blocks (W4 groups of 128 at
+//   32,768 tokens 2.67 ms against 2.73 with eighths).
 struct Placement {
     uint32_t task, slice;
 };
 
 constexpr uint32_t kXcds = 8;
 constexpr uint32_t kTaskBlock = 4;
+constexpr uint32_t kBlockedSlots = 2048;
+
+// the task slots a launch covers
+struct TaskSlots {
+    const q38m_task_v1* tasks;
+    const uint32_t* live;  // the plan's task count for contiguous eighths, null for blocks
+    uint32_t count;
+};
 
 __host__ __device__ constexpr uint32_t placed_workgroups(uint32_t task_slots, uint32_t slices) {
     constexpr uint32_t kRound = kXcds * kTaskBlock;
     return (task_slots + kRound - 1u) / kRound * kRound * slices;
 }
 
-__device__ inline bool place_on_xcds(uint32_t task_slots, uint32_t slices, Placement& at) {
+__device__ inline bool place_on_xcds(const TaskSlots& t, uint32_t slices, Placement& at) {
     const uint32_t xcd = blockIdx.x % kXcds, j = blockIdx.x / kXcds;
+    if (t.live != nullptr) {
+        const uint32_t pairs = min(*t.live, t.count) * slices;
+        const uint32_t per = pairs / kXcds, extra = pairs % kXcds;
+        if (j >= per + (xcd < extra ? 1u : 0u)) return false;
+        const uint32_t pair = xcd * per + min(xcd, extra) + j;
+        at.task = pair / slices;
+        at.slice = pair % slices;
+        return true;
+    }
     const uint32_t within = j % (kTaskBlock * slices);
     at.task = (j / (kTaskBlock * slices) * kXcds + xcd) * kTaskBlock + within / slices;
     at.slice = within % slices;
-    return at.task < task_slots;
+    return at.task < t.count;
 }
 
 // ---- gate/up ----------------------------------------------------------------
@@ -434,8 +459,7 @@ void gate_up_w4g32_f16_kernel(const uint4* __restrict__ w, const uint16_t* __res
                               const int8_t* __restrict__ xq, const float* __restrict__ xs,
                               const uint32_t* __restrict__ packed,
                               const float* __restrict__ route_weights,
-                              const q38m_task_v1* __restrict__ tasks,
-                              uint32_t task_slots, uint16_t* __restrict__ mid) {
+                              TaskSlots slots, uint16_t* __restrict__ mid) {
     constexpr uint32_t kHalves = H / 64u;  // staging steps
     constexpr uint32_t kTilesAll = 2u * I / 16u;
     constexpr uint32_t kWgTiles = 16u;  // 8 pairs
@@ -449,8 +473,8 @@ void gate_up_w4g32_f16_kernel(const uint4* __restrict__ w, const uint16_t* __res
     __shared__ float2 row_info[kWideRows];  // (token scale, route weight)
 
     Placement at;
-    if (!place_on_xcds(task_slots, I / 16u / 8u, at)) return;
-    const TaskRecord task = read_task(tasks, at.task);
+    if (!place_on_xcds(slots, I / 16u / 8u, at)) return;
+    const TaskRecord task = read_task(slots.tasks, at.task);
     const uint32_t rows = task.rows;
     if (rows == 0u) return;
     const uint32_t tid = threadIdx.x;
@@ -736,7 +760,7 @@ template <uint32_t H, uint32_t I, uint32_t kWaves, uint32_t kTilesPerWave, bool 
 __global__ __launch_bounds__(kWaves * 64) void down_w8_wide_kernel(
     const uint4* __restrict__ w, const uint16_t* __restrict__ s,
     const int8_t* __restrict__ mq, const float* __restrict__ ms,
-    const q38m_task_v1* __restrict__ tasks, uint32_t task_slots, float* __restrict__ out) {
+    TaskSlots slots, float* __restrict__ out) {
     constexpr uint32_t kBlocks = I / 64u;
     constexpr uint32_t kTiles = H / 16u;
     constexpr uint32_t kThreads = kWaves * 64u;
@@ -746,8 +770,8 @@ __global__ __launch_bounds__(kWaves * 64) void down_w8_wide_kernel(
     __shared__ float row_scale[kWideRows];
 
     Placement at;
-    if (!place_on_xcds(task_slots, H / 16u / (kWaves * kTilesPerWave), at)) return;
-    const TaskRecord task = read_task(tasks, at.task);
+    if (!place_on_xcds(slots, H / 16u / (kWaves * kTilesPerWave), at)) return;
+    const TaskRecord task = read_task(slots.tasks, at.task);
     const uint32_t rows = task.rows;
     if (rows == 0u) return;
     const uint32_t lane = threadIdx.x & 63u;
@@ -811,8 +835,7 @@ template <uint32_t H, uint32_t I, bool kBf16>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
 void down_w4g32_f16_kernel(const uint4* __restrict__ w, const uint16_t* __restrict__ s,
                            const int8_t* __restrict__ mq, const float* __restrict__ ms,
-                           const q38m_task_v1* __restrict__ tasks,
-                           uint32_t task_slots, float* __restrict__ out) {
+                           TaskSlots slots, float* __restrict__ out) {
     constexpr uint32_t kSteps = I / 64u;
     constexpr uint32_t kTiles = H / 16u;
     static_assert(kSteps % 2u == 0u, "steps run in pairs of LDS buffers");
@@ -820,8 +843,8 @@ void down_w4g32_f16_kernel(const uint4* __restrict__ w, const uint16_t* __restri
     __shared__ float row_scale[kWideRows];
 
     Placement at;
-    if (!place_on_xcds(task_slots, H / 16u / 16u, at)) return;
-    const TaskRecord task = read_task(tasks, at.task);
+    if (!place_on_xcds(slots, H / 16u / 16u, at)) return;
+    const TaskRecord task = read_task(slots.tasks, at.task);
     const uint32_t rows = task.rows;
     if (rows == 0u) return;
     const uint32_t tid = threadIdx.x;
@@ -1039,7 +1062,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 void wide_i8_kernel(const uint4* __restrict__ w, const uint16_t* __restrict__ s,
                     const int8_t* __restrict__ rows_q, const float* __restrict__ row_scales,
                     const uint32_t* __restrict__ packed, const float* __restrict__ route_weights,
-                    const q38m_task_v1* __restrict__ tasks, uint32_t task_slots, void* __restrict__ out) {
+                    TaskSlots slots, void* __restrict__ out) {
     using F = WideI8<kBits, kGroup, kGateUp>;
     constexpr uint32_t kK = F::kK, kSlots = F::kSlots, kSteps = F::kSteps;
     static_assert(kSteps % 2u == 0u, "steps run in pairs of LDS buffers");
@@ -1048,8 +1071,8 @@ void wide_i8_kernel(const uint4* __restrict__ w, const uint16_t* __restrict__ s,
     __shared__ float2 row_info[kI8Rows];  // (row scale, route weight)
 
     Placement at;
-    if (!place_on_xcds(task_slots, F::kSlices * F::kHalves, at)) return;
-    const TaskRecord task = read_task(tasks, at.task);
+    if (!place_on_xcds(slots, F::kSlices * F::kHalves, at)) return;
+    const TaskRecord task = read_task(slots.tasks, at.task);
     // this workgroup's rows of the task: 64 from row 64 * half
     const uint32_t half = at.slice / F::kSlices;
     const uint32_t slice = at.slice % F::kSlices;
@@ -1376,12 +1399,6 @@ hipError_t launch_step_wide_plan(const int32_t* ids, uint32_t tokens,
 
 namespace {
 
-// the task slots a launch covers
-struct TaskSlots {
-    const q38m_task_v1* tasks;
-    uint32_t count;
-};
-
 template <uint32_t kBits, uint32_t kGroup, bool kBf16>
 void launch_gate_up_i8(const q38m_expert_weights_v1& w, const int8_t* xq, const float* xs,
                        const uint32_t* packed, const float* route_weights, const TaskSlots& t,
@@ -1390,7 +1407,7 @@ void launch_gate_up_i8(const q38m_expert_weights_v1& w, const int8_t* xq, const 
     const uint32_t grid = placed_workgroups(t.count, F::kSlices * F::kHalves);
     wide_i8_kernel<kBits, kGroup, kBf16, true><<<grid, 256, 0, stream>>>(
         static_cast<const uint4*>(w.data), static_cast<const uint16_t*>(w.scales), xq, xs, packed,
-        route_weights, t.tasks, t.count, mid);
+        route_weights, TaskSlots{t.tasks, nullptr, t.count}, mid);
 }
 
 template <uint32_t kBits, uint32_t kGroup, bool kBf16>
@@ -1400,7 +1417,7 @@ void launch_down_i8(const q38m_expert_weights_v1& w, const int8_t* mid_q, const 
     const uint32_t grid = placed_workgroups(t.count, F::kSlices * F::kHalves);
     wide_i8_kernel<kBits, kGroup, kBf16, false><<<grid, 256, 0, stream>>>(
         static_cast<const uint4*>(w.data), static_cast<const uint16_t*>(w.scales), mid_q, mid_s,
-        nullptr, nullptr, t.tasks, t.count, route_output);
+        nullptr, nullptr, TaskSlots{t.tasks, nullptr, t.count}, route_output);
 }
 
 template <bool kBf16>
@@ -1415,7 +1432,7 @@ hipError_t launch_gate_up_wide_dtype(const q38m_expert_weights_v1& w, const int8
             const uint32_t grid = placed_workgroups(t.count, kInter / 16u / 8u);
             gate_up_w4g32_f16_kernel<kHidden, kInter, kBf16><<<grid, 512, 0, stream>>>(
                 static_cast<const uint4*>(w.data), static_cast<const uint16_t*>(w.scales), xq, xs,
-                packed, route_weights, t.tasks, t.count, mid);
+                packed, route_weights, t, mid);
             break;
         }
         case 4064u: launch_gate_up_i8<4, 64, kBf16>(w, xq, xs, packed, route_weights, t, mid, stream); break;
@@ -1439,7 +1456,7 @@ hipError_t launch_down_wide_dtype(const q38m_expert_weights_v1& w, const int8_t*
             const uint32_t grid = placed_workgroups(t.count, kHidden / 16u / 16u);
             down_w4g32_f16_kernel<kHidden, kInter, kBf16><<<grid, 512, 0, stream>>>(
                 static_cast<const uint4*>(w.data), static_cast<const uint16_t*>(w.scales), mid_q,
-                mid_s, t.tasks, t.count, out);
+                mid_s, t, out);
             break;
         }
         case 4064u: launch_down_i8<4, 64, kBf16>(w, mid_q, mid_s, t, out, stream); break;
@@ -1451,7 +1468,7 @@ hipError_t launch_down_wide_dtype(const q38m_expert_weights_v1& w, const int8_t*
             down_w8_wide_kernel<kHidden, kInter, kWaves, kTilesPerWave, kBf16>
                 <<<grid, kWaves * 64u, 0, stream>>>(static_cast<const uint4*>(w.data),
                                                     static_cast<const uint16_t*>(w.scales), mid_q,
-                                                    mid_s, t.tasks, t.count, out);
+                                                    mid_s, t, out);
             break;
         }
         case 8064u: launch_down_i8<8, 64, kBf16>(w, mid_q, mid_s, t, out, stream); break;
@@ -1465,8 +1482,10 @@ hipError_t launch_down_wide_dtype(const q38m_expert_weights_v1& w, const int8_t*
 
 hipError_t launch_gate_up_wide(const q38m_expert_weights_v1& w, const int8_t* xq, const float* xs,
                                const uint32_t* packed, const float* route_weights,
-                               const q38m_task_v1* tasks, uint32_t task_count, uint16_t* weighted_mid, hipStream_t stream) {
-    const TaskSlots t{tasks, task_count};
+                               const q38m_task_v1* tasks, const uint32_t* live_tasks,
+                               uint32_t task_count, uint16_t* weighted_mid,
+                               hipStream_t stream) {
+    const TaskSlots t{tasks, task_count > kBlockedSlots ? live_tasks : nullptr, task_count};
     return w.scale_dtype == Q38M_SCALE_BF16
                ? launch_gate_up_wide_dtype<true>(w, xq, xs, packed, route_weights, t,
                                                  weighted_mid, stream)
@@ -1475,9 +1494,10 @@ hipError_t launch_gate_up_wide(const q38m_expert_weights_v1& w, const int8_t* xq
 }
 
 hipError_t launch_down_wide(const q38m_expert_weights_v1& w, const int8_t* mid_q,
-                            const float* mid_s, const q38m_task_v1* tasks, uint32_t task_count,
+                            const float* mid_s, const q38m_task_v1* tasks,
+                            const uint32_t* live_tasks, uint32_t task_count,
                             float* route_output, hipStream_t stream) {
-    const TaskSlots t{tasks, task_count};
+    const TaskSlots t{tasks, task_count > kBlockedSlots ? live_tasks : nullptr, task_count};
     return w.scale_dtype == Q38M_SCALE_BF16
                ? launch_down_wide_dtype<true>(w, mid_q, mid_s, t, route_output, stream)
                : launch_down_wide_dtype<false>(w, mid_q, mid_s, t, route_output, stream);
