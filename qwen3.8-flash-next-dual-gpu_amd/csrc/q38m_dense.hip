@@ -14,6 +14,7 @@
 #include "q38m_device.h"
 #include "q38m_internal.h"
 #include "q38m_select.h"
+#include "q38m_tiles.h"
 
 namespace q38m {
 namespace {
@@ -615,9 +616,13 @@ struct TileShape {
     static constexpr uint32_t kLoads = kRows / 32u;    // load instructions per wave and chunk
     static constexpr uint32_t kI = kTM / 32u;          // a wave's row tiles
     static constexpr uint32_t kJ = kTN / 32u / kNB;    // its column tiles per matrix
+    static constexpr uint32_t kColumns = kTN / kNB;    // the workgroup's columns per matrix
     // all of a chunk's fragments in registers at once (beside 128 x 128 x 2
     // matrices' accumulators and totals they would spill)
     static constexpr bool kWholeChunk = kTM + kTN * kNB <= 256u;
+
+    static constexpr uint32_t row_tiles(uint32_t m) { return (m + kTM - 1u) / kTM; }
+    static constexpr uint32_t column_tiles(uint32_t n) { return (n + kColumns - 1u) / kColumns; }
 };
 
 // 16 bytes per lane from `src` (each lane its own) to the 1 KB at `lds`
@@ -823,27 +828,13 @@ __device__ __forceinline__ void tile_product(const uint16_t* __restrict__ a,
     }
 }
 
-// Tile of a one-dimensional grid: XCD x (workgroups x, x + 8, ...) runs row
-// tiles x, x + 8, ..., all column tiles of one before the next, so that a row
-// tile's activations are fetched into one L2.
-struct TileAt {
-    uint32_t row, column;
-};
-__device__ __forceinline__ TileAt tile_at(uint32_t column_tiles) {
-    const uint32_t j = blockIdx.x / 8u;
-    return TileAt{j / column_tiles * 8u + blockIdx.x % 8u, j % column_tiles};
-}
-constexpr uint32_t tile_grid(uint32_t row_tiles, uint32_t column_tiles) {
-    return (row_tiles + 7u) / 8u * 8u * column_tiles;
-}
-
 template <typename S, bool kSplit, DenseOut kOut>
 __global__ __launch_bounds__(256, 2) void dense_tile_kernel(
     const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint32_t m, uint32_t n,
     uint32_t k, float* __restrict__ c_f32, uint16_t* __restrict__ c_bf16, float divisor,
     float scale) {
     __shared__ u32x4 ring[S::kStages * S::kSlot];
-    const TileAt at = tile_at((n + S::kTN - 1u) / S::kTN);
+    const TileAt at = tile_at(blockIdx.x, (n + S::kTN - 1u) / S::kTN);
     const uint32_t m0 = at.row * S::kTM, n0 = at.column * S::kTN;
     if (m0 >= m) return;
     tile_product<S, kSplit, false>(
@@ -871,7 +862,7 @@ __global__ __launch_bounds__(256, 2) void shared_gate_up_tile_kernel(
     __shared__ u32x4 gate_lds[kHidden / 8u];
     static_assert(kHidden / 8u == 256u, "one vector of the gate row per thread");
     constexpr uint32_t kChannels = S::kTN / 2u;
-    const TileAt at = tile_at((inter + kChannels - 1u) / kChannels);
+    const TileAt at = tile_at(blockIdx.x, (inter + kChannels - 1u) / kChannels);
     const uint32_t m0 = at.row * S::kTM, n0 = at.column * kChannels;
     if (m0 >= m) return;
     auto finish = [&](uint32_t row, uint32_t col, const float (&v)[2], bool gate) {
@@ -910,7 +901,7 @@ __global__ __launch_bounds__(256, 2) void dense_quarter_kernel(const uint16_t* _
                                                                uint32_t m, uint32_t n, uint32_t k,
                                                                float* __restrict__ partials) {
     __shared__ u32x4 ring[S::kStages * S::kSlot];
-    const TileAt at = tile_at((n + S::kTN - 1u) / S::kTN);
+    const TileAt at = tile_at(blockIdx.x, (n + S::kTN - 1u) / S::kTN);
     const uint32_t m0 = at.row * S::kTM, n0 = at.column * S::kTN;
     if (m0 >= m) return;
     const uint32_t q = blockIdx.y, span = k / 4u;
@@ -975,7 +966,7 @@ __global__ __launch_bounds__(256, 2) void hyper_mix_up_kernel(
     // by pairs of column tiles (the halves of 128-byte lines): an XCD runs
     // every token tile of a pair before the next pair, so that mix_up's rows
     // are fetched into one L2
-    const TileAt at = tile_at(2u * ((tokens + kTokens - 1u) / kTokens));
+    const TileAt at = tile_at(blockIdx.x, 2u * ((tokens + kTokens - 1u) / kTokens));
     const uint32_t t0 = at.column / 2u * kTokens;
     const uint32_t c0 = (2u * at.row + at.column % 2u) * kChannels;
     if (c0 >= hidden) return;
@@ -1152,12 +1143,15 @@ namespace {
 constexpr uint32_t kGemvMaxRows = 65535u * 4u;
 
 template <typename S, bool kSplit, DenseOut kOut>
-void launch_dense_tile(const uint16_t* a, const uint16_t* b, uint32_t m, uint32_t n, uint32_t k,
+bool launch_dense_tile(const uint16_t* a, const uint16_t* b, uint32_t m, uint32_t n, uint32_t k,
                        float* c_f32, uint16_t* c_bf16, float divisor, float scale,
                        hipStream_t stream) {
+    const uint32_t rows = S::row_tiles(m), columns = S::column_tiles(n);
+    if (!tile_grid_fits(rows, columns)) return false;
     dense_tile_kernel<S, kSplit, kOut>
-        <<<tile_grid((m + S::kTM - 1u) / S::kTM, (n + S::kTN - 1u) / S::kTN), 256, 0, stream>>>(
+        <<<static_cast<uint32_t>(tile_grid(rows, columns)), 256, 0, stream>>>(
             a, b, m, n, k, c_f32, c_bf16, divisor, scale);
+    return true;
 }
 
 void launch_shared_small(const uint16_t* hidden, const uint16_t* w_gate, const uint16_t* w_up,
@@ -1169,13 +1163,15 @@ void launch_shared_small(const uint16_t* hidden, const uint16_t* w_gate, const u
 }
 
 template <typename S>
-void launch_shared_tile(const uint16_t* hidden, const uint16_t* w_gate, const uint16_t* w_up,
+bool launch_shared_tile(const uint16_t* hidden, const uint16_t* w_gate, const uint16_t* w_up,
                         const uint16_t* w_out_gate, uint32_t tokens, uint32_t inter, uint16_t* g,
                         uint16_t* u, uint16_t* h, uint16_t* gate, hipStream_t stream) {
-    constexpr uint32_t kChannels = S::kTN / 2u;
+    const uint32_t rows = S::row_tiles(tokens), columns = S::column_tiles(inter);
+    if (!tile_grid_fits(rows, columns)) return false;
     shared_gate_up_tile_kernel<S>
-        <<<tile_grid((tokens + S::kTM - 1u) / S::kTM, (inter + kChannels - 1u) / kChannels), 256, 0,
-           stream>>>(hidden, w_gate, w_up, w_out_gate, tokens, inter, g, u, h, gate);
+        <<<static_cast<uint32_t>(tile_grid(rows, columns)), 256, 0, stream>>>(
+            hidden, w_gate, w_up, w_out_gate, tokens, inter, g, u, h, gate);
+    return true;
 }
 
 // Large products take workgroup tiles: 64 x 64 with three chunks in the ring
@@ -1189,8 +1185,6 @@ void launch_shared_tile(const uint16_t* hidden, const uint16_t* w_gate, const ui
 // rows 20.5 / 16.9 / 17.9, 32,768 rows 125 / 136 / 101.
 constexpr uint32_t kTileMinTiles = 192;
 constexpr uint32_t kTile128MinTiles = 384;
-// their one-dimensional grids hold at most 2^32 threads
-constexpr uint64_t kTileMaxTiles = (1ull << 23);
 template <uint32_t kNB>
 using Tile64 = TileShape<64, 64, kNB, 3>;
 template <uint32_t kNB>
@@ -1209,18 +1203,13 @@ bool launch_dense_large(const uint16_t* a, const uint16_t* b, uint32_t m, uint32
                         float* c_f32, uint16_t* c_bf16, float divisor, float scale,
                         hipStream_t stream) {
     // whole chunks, for the split in every quarter, and as many as a ring's
-    if (k % (kSplit ? 256u : 64u) != 0u || k < 3u * 64u ||
-        tile_count(m, n, 64u, 64u) > kTileMaxTiles)
-        return false;
+    if (k % (kSplit ? 256u : 64u) != 0u || k < 3u * 64u) return false;
     if (tile_count(m, n, 128u, 128u) >= kTile128MinTiles)
-        launch_dense_tile<Tile128<1>, kSplit, kOut>(a, b, m, n, k, c_f32, c_bf16, divisor, scale,
-                                                    stream);
-    else if (tile_count(m, n, 64u, 64u) >= kTileMinTiles)
-        launch_dense_tile<Tile64<1>, kSplit, kOut>(a, b, m, n, k, c_f32, c_bf16, divisor, scale,
-                                                   stream);
-    else
-        return false;
-    return true;
+        return launch_dense_tile<Tile128<1>, kSplit, kOut>(a, b, m, n, k, c_f32, c_bf16, divisor,
+                                                           scale, stream);
+    return tile_count(m, n, 64u, 64u) >= kTileMinTiles &&
+           launch_dense_tile<Tile64<1>, kSplit, kOut>(a, b, m, n, k, c_f32, c_bf16, divisor,
+                                                      scale, stream);
 }
 
 template <DenseOut kOut>
@@ -1300,8 +1289,8 @@ bool launch_hyper_mix_down(const uint16_t* x, const uint16_t* mix_down, uint32_t
     if (tokens < kHyperTileMinTokens || tiles >= 512u || width % 256u != 0u ||
         width / 256u < S::kStages || (static_cast<uint64_t>(tokens) * rank) % 4u != 0u)
         return false;
-    dense_quarter_kernel<S>
-        <<<dim3(tile_grid((tokens + 63u) / 64u, (rank + 63u) / 64u), 4), 256, 0, stream>>>(
+    const uint64_t grid = tile_grid(S::row_tiles(tokens), S::column_tiles(rank));
+    dense_quarter_kernel<S><<<dim3(static_cast<uint32_t>(grid), 4), 256, 0, stream>>>(
             x, mix_down, tokens, rank, width, partials);
     const uint32_t total4 = tokens * rank / 4u;
     quarter_silu_kernel<<<(total4 + 255u) / 256u, 256, 0, stream>>>(
@@ -1313,14 +1302,13 @@ bool launch_hyper_mix_down(const uint16_t* x, const uint16_t* mix_down, uint32_t
 bool launch_hyper_mix_up(const uint16_t* low, const uint16_t* mix_up, const uint16_t* normalized,
                          uint32_t tokens, uint32_t hidden, uint32_t rank, uint16_t* mixed,
                          hipStream_t stream, hipError_t* status) {
-    const uint64_t workgroups = (static_cast<uint64_t>(tokens) + 127u) / 128u * (hidden / 32u);
+    const uint32_t rows = (hidden + 63u) / 64u, columns = 2u * ((tokens + 127u) / 128u);
     // the shapes whose product runs over one accumulator (launch_dense_tiles)
     if (tokens < kHyperTileMinTokens || hidden % 32u != 0u || rank % 32u != 0u ||
         rank > kTile64MaxK || tile_count(tokens, 4u * hidden, 64u, 64u) < kTile64MinTiles ||
-        workgroups > kTileMaxTiles)
+        !tile_grid_fits(rows, columns))
         return false;
-    hyper_mix_up_kernel<<<tile_grid((hidden + 63u) / 64u, 2u * ((tokens + 127u) / 128u)), 256, 0,
-                          stream>>>(
+    hyper_mix_up_kernel<<<static_cast<uint32_t>(tile_grid(rows, columns)), 256, 0, stream>>>(
         low, mix_up, normalized, tokens, hidden, rank, mixed);
     *status = hipGetLastError();
     return true;
@@ -1377,16 +1365,16 @@ hipError_t launch_shared_expert(const uint16_t* hidden, const uint16_t* w_gate,
         shared_gate_up_gemv_kernel<<<(inter + 2u) / 2u, 128, 0, stream>>>(
             hidden, w_gate, w_up, w_out_gate, inter, g, u, h, shared_gate);
     } else {
-        const uint64_t tiles64 = tile_count(tokens, 2u * inter, 64u, 64u);
-        if (tiles64 < kTileMinTiles || tiles64 > kTileMaxTiles)
+        bool done = false;
+        if (tile_count(tokens, 2u * inter, 128u, 128u) >= kTile128MinTiles)
+            done = launch_shared_tile<Tile128<2>>(hidden, w_gate, w_up, w_out_gate, tokens, inter,
+                                                  g, u, h, shared_gate, stream);
+        else if (tile_count(tokens, 2u * inter, 64u, 64u) >= kTileMinTiles)
+            done = launch_shared_tile<Tile64<2>>(hidden, w_gate, w_up, w_out_gate, tokens, inter,
+                                                 g, u, h, shared_gate, stream);
+        if (!done)
             launch_shared_small(hidden, w_gate, w_up, w_out_gate, tokens, inter, g, u, h,
                                 shared_gate, stream);
-        else if (tile_count(tokens, 2u * inter, 128u, 128u) < kTile128MinTiles)
-            launch_shared_tile<Tile64<2>>(hidden, w_gate, w_up, w_out_gate, tokens, inter, g, u, h,
-                                          shared_gate, stream);
-        else
-            launch_shared_tile<Tile128<2>>(hidden, w_gate, w_up, w_out_gate, tokens, inter, g, u,
-                                           h, shared_gate, stream);
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
