@@ -832,9 +832,9 @@ template <typename S, bool kSplit, DenseOut kOut>
 __global__ __launch_bounds__(256, 2) void dense_tile_kernel(
     const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint32_t m, uint32_t n,
     uint32_t k, float* __restrict__ c_f32, uint16_t* __restrict__ c_bf16, float divisor,
-    float scale) {
+    float scale, TileOrder order) {
     __shared__ u32x4 ring[S::kStages * S::kSlot];
-    const TileAt at = tile_at(blockIdx.x, (n + S::kTN - 1u) / S::kTN);
+    const TileAt at = tile_at(blockIdx.x, order, S::row_tiles(m), S::column_tiles(n));
     const uint32_t m0 = at.row * S::kTM, n0 = at.column * S::kTN;
     if (m0 >= m) return;
     tile_product<S, kSplit, false>(
@@ -857,13 +857,12 @@ __global__ __launch_bounds__(256, 2) void shared_gate_up_tile_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ w_gate,
     const uint16_t* __restrict__ w_up, const uint16_t* __restrict__ w_out_gate, uint32_t m,
     uint32_t inter, uint16_t* __restrict__ g_out, uint16_t* __restrict__ u_out,
-    uint16_t* __restrict__ h_out, uint16_t* __restrict__ gate_out) {
+    uint16_t* __restrict__ h_out, uint16_t* __restrict__ gate_out, TileOrder order) {
     __shared__ u32x4 ring[S::kStages * S::kSlot];
     __shared__ u32x4 gate_lds[kHidden / 8u];
     static_assert(kHidden / 8u == 256u, "one vector of the gate row per thread");
-    constexpr uint32_t kChannels = S::kTN / 2u;
-    const TileAt at = tile_at(blockIdx.x, (inter + kChannels - 1u) / kChannels);
-    const uint32_t m0 = at.row * S::kTM, n0 = at.column * kChannels;
+    const TileAt at = tile_at(blockIdx.x, order, S::row_tiles(m), S::column_tiles(inter));
+    const uint32_t m0 = at.row * S::kTM, n0 = at.column * S::kColumns;
     if (m0 >= m) return;
     auto finish = [&](uint32_t row, uint32_t col, const float (&v)[2], bool gate) {
         if (row >= m) return;
@@ -899,9 +898,10 @@ template <typename S>
 __global__ __launch_bounds__(256, 2) void dense_quarter_kernel(const uint16_t* __restrict__ a,
                                                                const uint16_t* __restrict__ b,
                                                                uint32_t m, uint32_t n, uint32_t k,
-                                                               float* __restrict__ partials) {
+                                                               float* __restrict__ partials,
+                                                               TileOrder order) {
     __shared__ u32x4 ring[S::kStages * S::kSlot];
-    const TileAt at = tile_at(blockIdx.x, (n + S::kTN - 1u) / S::kTN);
+    const TileAt at = tile_at(blockIdx.x, order, S::row_tiles(m), S::column_tiles(n));
     const uint32_t m0 = at.row * S::kTM, n0 = at.column * S::kTN;
     if (m0 >= m) return;
     const uint32_t q = blockIdx.y, span = k / 4u;
@@ -956,7 +956,7 @@ __device__ const uint32_t kSigmoidTable[4096] = {
 __global__ __launch_bounds__(256, 2) void hyper_mix_up_kernel(
     const uint16_t* __restrict__ low, const uint16_t* __restrict__ up,
     const uint16_t* __restrict__ normalized, uint32_t tokens, uint32_t hidden, uint32_t rank,
-    uint16_t* __restrict__ mixed) {
+    uint16_t* __restrict__ mixed, TileOrder order) {
     constexpr uint32_t kStreams = 4, kTokens = 128, kChannels = 32, kStages = 2;
     constexpr uint32_t kJ = kTokens / 64u;  // a wave's token tiles
     constexpr uint32_t kRows = kStreams * kChannels + kTokens;
@@ -966,7 +966,8 @@ __global__ __launch_bounds__(256, 2) void hyper_mix_up_kernel(
     // by pairs of column tiles (the halves of 128-byte lines): an XCD runs
     // every token tile of a pair before the next pair, so that mix_up's rows
     // are fetched into one L2
-    const TileAt at = tile_at(blockIdx.x, 2u * ((tokens + kTokens - 1u) / kTokens));
+    const TileAt at = tile_at(blockIdx.x, order, (hidden + 2u * kChannels - 1u) / (2u * kChannels),
+                              2u * ((tokens + kTokens - 1u) / kTokens));
     const uint32_t t0 = at.column / 2u * kTokens;
     const uint32_t c0 = (2u * at.row + at.column % 2u) * kChannels;
     if (c0 >= hidden) return;
@@ -1147,10 +1148,11 @@ bool launch_dense_tile(const uint16_t* a, const uint16_t* b, uint32_t m, uint32_
                        float* c_f32, uint16_t* c_bf16, float divisor, float scale,
                        hipStream_t stream) {
     const uint32_t rows = S::row_tiles(m), columns = S::column_tiles(n);
-    if (!tile_grid_fits(rows, columns)) return false;
+    const TileOrder order = tile_order(rows, columns, 2ull * n * k, k);
+    if (!tile_grid_fits(order, rows, columns)) return false;
     dense_tile_kernel<S, kSplit, kOut>
-        <<<static_cast<uint32_t>(tile_grid(rows, columns)), 256, 0, stream>>>(
-            a, b, m, n, k, c_f32, c_bf16, divisor, scale);
+        <<<static_cast<uint32_t>(tile_grid(order, rows, columns)), 256, 0, stream>>>(
+            a, b, m, n, k, c_f32, c_bf16, divisor, scale, order);
     return true;
 }
 
@@ -1167,10 +1169,11 @@ bool launch_shared_tile(const uint16_t* hidden, const uint16_t* w_gate, const ui
                         const uint16_t* w_out_gate, uint32_t tokens, uint32_t inter, uint16_t* g,
                         uint16_t* u, uint16_t* h, uint16_t* gate, hipStream_t stream) {
     const uint32_t rows = S::row_tiles(tokens), columns = S::column_tiles(inter);
-    if (!tile_grid_fits(rows, columns)) return false;
+    const TileOrder order = tile_order(rows, columns, 4ull * inter * kHidden, kHidden);
+    if (!tile_grid_fits(order, rows, columns)) return false;
     shared_gate_up_tile_kernel<S>
-        <<<static_cast<uint32_t>(tile_grid(rows, columns)), 256, 0, stream>>>(
-            hidden, w_gate, w_up, w_out_gate, tokens, inter, g, u, h, gate);
+        <<<static_cast<uint32_t>(tile_grid(order, rows, columns)), 256, 0, stream>>>(
+            hidden, w_gate, w_up, w_out_gate, tokens, inter, g, u, h, gate, order);
     return true;
 }
 
@@ -1196,18 +1199,27 @@ constexpr uint64_t tile_count(uint32_t m, uint32_t n, uint32_t rows, uint32_t co
            ((static_cast<uint64_t>(n) + columns - 1u) / columns);
 }
 
-// the product on workgroup tiles where they are the faster form; kSplit: the
-// summation order of the kernel they stand in for
+// The product on workgroup tiles where they are the faster form; kSplit: the
+// summation order of the kernel they stand in for.  With K split that kernel
+// keeps up to 32 rows or columns, which its 16- and 32-row tiles fit, and up to
+// 512 rows below 200 tiles (us as that kernel / 64 x 64 / 128 x 128: 2 x 12,288
+// x 2,048 6.8 / 10.9 / 22.7, 32 rows 9.1 / 11.3 / 23.2, 48 rows 13.0 / 11.0 /
+// 23.5; 321 x 2,048 x 2,048 10.2 / 11.4 / 23.4).  128 x 128 tiles need more than
+// 64 rows and, over whole K, columns (64 x 151,936 x 2,048 255 / 137 / 162;
+// 131,072 x 64 x 320 16.1 / 16.4 / 20.4; K split, 65,536 x 64 x 2,048 72.9 / 47.0
+// / 43.8).
 template <bool kSplit, DenseOut kOut>
 bool launch_dense_large(const uint16_t* a, const uint16_t* b, uint32_t m, uint32_t n, uint32_t k,
                         float* c_f32, uint16_t* c_bf16, float divisor, float scale,
                         hipStream_t stream) {
     // whole chunks, for the split in every quarter, and as many as a ring's
     if (k % (kSplit ? 256u : 64u) != 0u || k < 3u * 64u) return false;
-    if (tile_count(m, n, 128u, 128u) >= kTile128MinTiles)
+    const uint64_t tiles64 = tile_count(m, n, 64u, 64u);
+    if (kSplit && (m <= 32u || n <= 32u || (m <= 512u && tiles64 < 200u))) return false;
+    if (tile_count(m, n, 128u, 128u) >= kTile128MinTiles && m > 64u && (kSplit || n > 64u))
         return launch_dense_tile<Tile128<1>, kSplit, kOut>(a, b, m, n, k, c_f32, c_bf16, divisor,
                                                            scale, stream);
-    return tile_count(m, n, 64u, 64u) >= kTileMinTiles &&
+    return tiles64 >= kTileMinTiles &&
            launch_dense_tile<Tile64<1>, kSplit, kOut>(a, b, m, n, k, c_f32, c_bf16, divisor,
                                                       scale, stream);
 }
@@ -1289,9 +1301,12 @@ bool launch_hyper_mix_down(const uint16_t* x, const uint16_t* mix_down, uint32_t
     if (tokens < kHyperTileMinTokens || tiles >= 512u || width % 256u != 0u ||
         width / 256u < S::kStages || (static_cast<uint64_t>(tokens) * rank) % 4u != 0u)
         return false;
-    const uint64_t grid = tile_grid(S::row_tiles(tokens), S::column_tiles(rank));
-    dense_quarter_kernel<S><<<dim3(static_cast<uint32_t>(grid), 4), 256, 0, stream>>>(
-            x, mix_down, tokens, rank, width, partials);
+    const uint32_t span = width / 4u;
+    const uint32_t rows = S::row_tiles(tokens), columns = S::column_tiles(rank);
+    const TileOrder order = tile_order(rows, columns, 2ull * rank * span, span);
+    dense_quarter_kernel<S>
+        <<<dim3(static_cast<uint32_t>(tile_grid(order, rows, columns)), 4), 256, 0, stream>>>(
+            x, mix_down, tokens, rank, width, partials, order);
     const uint32_t total4 = tokens * rank / 4u;
     quarter_silu_kernel<<<(total4 + 255u) / 256u, 256, 0, stream>>>(
         reinterpret_cast<const f32x4*>(partials), total4, divisor, low);
@@ -1303,13 +1318,14 @@ bool launch_hyper_mix_up(const uint16_t* low, const uint16_t* mix_up, const uint
                          uint32_t tokens, uint32_t hidden, uint32_t rank, uint16_t* mixed,
                          hipStream_t stream, hipError_t* status) {
     const uint32_t rows = (hidden + 63u) / 64u, columns = 2u * ((tokens + 127u) / 128u);
+    const TileOrder order = tile_order(rows, columns, 0u, rank);
     // the shapes whose product runs over one accumulator (launch_dense_tiles)
     if (tokens < kHyperTileMinTokens || hidden % 32u != 0u || rank % 32u != 0u ||
         rank > kTile64MaxK || tile_count(tokens, 4u * hidden, 64u, 64u) < kTile64MinTiles ||
-        !tile_grid_fits(rows, columns))
+        !tile_grid_fits(order, rows, columns))
         return false;
-    hyper_mix_up_kernel<<<static_cast<uint32_t>(tile_grid(rows, columns)), 256, 0, stream>>>(
-        low, mix_up, normalized, tokens, hidden, rank, mixed);
+    hyper_mix_up_kernel<<<static_cast<uint32_t>(tile_grid(order, rows, columns)), 256, 0, stream>>>(
+        low, mix_up, normalized, tokens, hidden, rank, mixed, order);
     *status = hipGetLastError();
     return true;
 }
@@ -1365,13 +1381,19 @@ hipError_t launch_shared_expert(const uint16_t* hidden, const uint16_t* w_gate,
         shared_gate_up_gemv_kernel<<<(inter + 2u) / 2u, 128, 0, stream>>>(
             hidden, w_gate, w_up, w_out_gate, inter, g, u, h, shared_gate);
     } else {
+        // (up to 32 tokens half of a tile's rows repeat the last token: 2
+        // tokens, inter 6,144 17.6 us on the small tiles, 18.5 here; 8,192
+        // 21.6 / 20.8, 16,384 37.8 / 34.4)
+        const uint64_t tiles64 = tile_count(tokens, 2u * inter, 64u, 64u);
         bool done = false;
-        if (tile_count(tokens, 2u * inter, 128u, 128u) >= kTile128MinTiles)
-            done = launch_shared_tile<Tile128<2>>(hidden, w_gate, w_up, w_out_gate, tokens, inter,
-                                                  g, u, h, shared_gate, stream);
-        else if (tile_count(tokens, 2u * inter, 64u, 64u) >= kTileMinTiles)
-            done = launch_shared_tile<Tile64<2>>(hidden, w_gate, w_up, w_out_gate, tokens, inter,
-                                                 g, u, h, shared_gate, stream);
+        if (tiles64 >= (tokens <= 32u ? 256u : kTileMinTiles)) {
+            if (tokens > 64u && tile_count(tokens, 2u * inter, 128u, 128u) >= kTile128MinTiles)
+                done = launch_shared_tile<Tile128<2>>(hidden, w_gate, w_up, w_out_gate, tokens,
+                                                      inter, g, u, h, shared_gate, stream);
+            else
+                done = launch_shared_tile<Tile64<2>>(hidden, w_gate, w_up, w_out_gate, tokens,
+                                                     inter, g, u, h, shared_gate, stream);
+        }
         if (!done)
             launch_shared_small(hidden, w_gate, w_up, w_out_gate, tokens, inter, g, u, h,
                                 shared_gate, stream);
