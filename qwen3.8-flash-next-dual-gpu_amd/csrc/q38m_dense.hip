@@ -1200,23 +1200,37 @@ constexpr uint64_t tile_count(uint32_t m, uint32_t n, uint32_t rows, uint32_t co
 }
 
 // The product on workgroup tiles where they are the faster form; kSplit: the
-// summation order of the kernel they stand in for.  With K split that kernel
-// keeps up to 32 rows or columns, which its 16- and 32-row tiles fit, and up to
-// 512 rows below 200 tiles (us as that kernel / 64 x 64 / 128 x 128: 2 x 12,288
-// x 2,048 6.8 / 10.9 / 22.7, 32 rows 9.1 / 11.3 / 23.2, 48 rows 13.0 / 11.0 /
-// 23.5; 321 x 2,048 x 2,048 10.2 / 11.4 / 23.4).  128 x 128 tiles need more than
-// 64 rows and, over whole K, columns (64 x 151,936 x 2,048 255 / 137 / 162;
-// 131,072 x 64 x 320 16.1 / 16.4 / 20.4; K split, 65,536 x 64 x 2,048 72.9 / 47.0
-// / 43.8).
+// summation order of the kernel they stand in for, which keeps (us as that
+// kernel / 64 x 64 / 128 x 128):
+// - with K split, up to 32 rows or columns, which its 16- and 32-row tiles fit
+//   (2 x 12,288 x 2,048 6.8 / 10.9 / 22.7, 32 rows 9.1 / 11.3 / 23.2, 48 rows
+//   13.0 / 11.0 / 23.5), and up to 512 rows below 200 tiles (321 x 2,048 x
+//   2,048 10.2 / 11.4 / 23.4);
+// - whole K of three or four chunks, which hardly fill the ring, beside many
+//   columns (4,099 x 16,384 x 192 57.0 / 79.5 / 63.6; x 320 83.5 / 87.1 / 74.4;
+//   16,384 x 12,000 x 192 238 / - / 172), five to seven chunks of up to 64 rows
+//   (2 x 65,536 x 320 7.6 / 8.4 / -; x 512 10.6 / 10.6 / -).
+// 128 x 128 tiles need more than 64 rows and, over whole K, columns (64 x
+// 151,936 x 2,048 255 / 137 / 162; 131,072 x 64 x 320 16.1 / 16.4 / 20.4; K
+// split, 65,536 x 64 x 2,048 72.9 / 47.0 / 43.8).  Two of them fit a CU: short
+// products of just over 512 run a second, nearly empty round (4,099 x 2,048 x
+// 192, 528 tiles, 9.4 / 9.2 / 10.5; x 512 17.6 / 15.6 / 17.9; 5,000 rows, 640
+// tiles, x 320 16.1 / 14.7 / 14.2).
 template <bool kSplit, DenseOut kOut>
 bool launch_dense_large(const uint16_t* a, const uint16_t* b, uint32_t m, uint32_t n, uint32_t k,
                         float* c_f32, uint16_t* c_bf16, float divisor, float scale,
                         hipStream_t stream) {
     // whole chunks, for the split in every quarter, and as many as a ring's
     if (k % (kSplit ? 256u : 64u) != 0u || k < 3u * 64u) return false;
-    const uint64_t tiles64 = tile_count(m, n, 64u, 64u);
-    if (kSplit && (m <= 32u || n <= 32u || (m <= 512u && tiles64 < 200u))) return false;
-    if (tile_count(m, n, 128u, 128u) >= kTile128MinTiles && m > 64u && (kSplit || n > 64u))
+    const uint64_t tiles64 = tile_count(m, n, 64u, 64u), tiles128 = tile_count(m, n, 128u, 128u);
+    bool tile128 = tiles128 >= kTile128MinTiles && m > 64u;
+    if constexpr (kSplit) {
+        if (m <= 32u || n <= 32u || (m <= 512u && tiles64 < 200u)) return false;
+    } else {
+        if (n >= 8192u && (m <= 64u ? k < 512u : k < 320u && m <= 8192u)) return false;
+        tile128 = tile128 && n > 64u && !(k <= 512u && tiles128 > 512u && tiles128 <= 608u);
+    }
+    if (tile128)
         return launch_dense_tile<Tile128<1>, kSplit, kOut>(a, b, m, n, k, c_f32, c_bf16, divisor,
                                                            scale, stream);
     return tiles64 >= kTileMinTiles &&

@@ -37,6 +37,25 @@ def test_whole_k_products(q38m, m, n, k):
     assert_close(gemm(q38m, a, b, False), a, b, False)
 
 
+@pytest.mark.parametrize("k,forms", [(192, ((8192, 16385), (4097, 4097), (9000, 16385))),
+                                     (320, ((64, 16385), (100, 16385), (700, 16385))),
+                                     (512, ((100, 16385), (400, 16385), (530, 12310))),
+                                     (1024, ((100, 16385), (400, 16385)))])
+def test_whole_k_forms_agree(q38m, k, forms):
+    """One accumulator over K in each form: the same words for the rows and
+    columns that the sizes share (k 192: the small tiles, 33 x 33 of 128 x 128,
+    71 x 129; k 320: the small tiles, 64 x 64, 128 x 128; k 512: 64 x 64, 64 x 64
+    where 128 x 128 would be 516 tiles, 128 x 128; k 1,024: 64 x 64, 128 x 128)."""
+    t = torch()
+    rows, columns = max(m for m, _ in forms), max(n for _, n in forms)
+    a, b = matrix(k, rows, k, 1.0), matrix(k + 1, columns, k, 0.04)
+    shared_rows, shared_columns = min(m for m, _ in forms), min(n for _, n in forms)
+    for bf16 in (False, True):
+        results = [gemm(q38m, a[:m], b[:n], bf16)[:shared_rows, :shared_columns] for m, n in forms]
+        for other in results[1:]:
+            assert t.equal(results[0], other)
+
+
 @pytest.mark.parametrize("tokens,inter", [(2, 8192), (32, 6144), (33, 6176), (100, 4096), (600, 4128)])
 def test_shared_expert_equals_channel_slices(q38m, tokens, inter):
     t = torch()
