@@ -23,6 +23,22 @@ def matrix(g, rows, columns, sigma):
     (1500, 2048, 288, True), (6500, 2048, 320, False), (520, 1000, 64, False),
     (600, 2080, 128, False)])
 def test_large_prepare_equals_small(q38m, tokens, hidden, rank, special):
+    assert_prepare_equals_slices(q38m, tokens, hidden, rank, special, 500)
+
+
+# past the line from which mix-down keeps K in one workgroup (512 tiles of 64 x
+# 64: 6,529 tokens at rank 320), and ranks above 1,024 (mix-down without
+# partials, mix-up with K split and the sigmoid in its epilogue, a separate
+# stream mix); slices of 500 tokens and of 30, whose products run on the
+# K-split kernels
+@pytest.mark.parametrize("tokens,hidden,rank", [(6600, 2048, 320), (6529, 2560, 320),
+                                                (1500, 2048, 1280), (2600, 2560, 1280)])
+@pytest.mark.parametrize("count", [500, 30])
+def test_prepare_past_the_quarters(q38m, tokens, hidden, rank, count):
+    assert_prepare_equals_slices(q38m, tokens, hidden, rank, False, count)
+
+
+def assert_prepare_equals_slices(q38m, tokens, hidden, rank, special, count):
     t = torch()
     g = t.Generator(device="cuda").manual_seed(tokens)
     wide = 4 * hidden
@@ -48,7 +64,7 @@ def test_large_prepare_equals_small(q38m, tokens, hidden, rank, special):
         return t.where(x.isnan(), t.full_like(x, float("nan")), x).view(t.int16)
 
     mixed, injection = run(state)
-    for rows in (slice(0, 500), slice(tokens - 500, tokens)):
+    for rows in (slice(0, count), slice(tokens - count, tokens)):
         small_mixed, small_injection = run(state[rows].contiguous())
         assert t.equal(words(mixed[rows]), words(small_mixed))
         assert t.equal(words(injection[rows]), words(small_injection))
