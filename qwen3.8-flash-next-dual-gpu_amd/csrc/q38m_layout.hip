@@ -146,8 +146,9 @@ __device__ __forceinline__ uint32_t f32_to_f16_bits(float v) {
 // The integers of eight bf16 values (four words) of a group with scale s,
 // r = RN(1/s), in the low kBits bits of each byte of (even values, odd
 // values).  Scales in [2^-120, FLT_MAX] take no division per value: one
-// Markstein correction step rounds like it for every bf16 pair
-// (tests/weight_quotient_check.c), and adding 1.5 * 2^23 rounds to the integer
+// Markstein correction step rounds like it (tests/weight_quotient_check.c walks
+// every bf16 pair of the lowest, middle and largest binades of maxima, between
+// which powers of two scale exactly), and adding 1.5 * 2^23 rounds to the integer
 // in the low bits; a NaN quotient clamps to -qmax on both paths.  (With
 // an IEEE division and a half-rate conversion per value the kernels moved
 // 3.5-4.4 TB/s, now 5.9-6.2.)
