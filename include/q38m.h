@@ -382,7 +382,7 @@ int q38m_moe_prefill_noalloc_v1(const q38m_expert_weights_v1* gate_up,
  * index); its tasks are 128-row tiles (header version 2). */
 typedef struct q38m_wide_workspace_v1 {
     q38m_prefill_workspace_v1 step; /* bound for max_tokens <= 32768 */
-    uint32_t* plan_scratch;         /* per-chunk expert counts */
+    uint32_t* plan_scratch;         /* scratch of q38m_moe_build_route_plan_wide */
 } q38m_wide_workspace_v1;
 
 /* Chunk plan alone: bytes of the plan views and of their build scratch. */
@@ -398,6 +398,10 @@ int q38m_moe_build_route_plan_wide(const int32_t* expert_ids, uint32_t tokens,
                                    const q38m_route_plan_v1* plan, uint32_t* scratch,
                                    void* stream, int device);
 
+/* One allocation for a chunk step.  plan_scratch is for a caller that builds
+ * the plan by itself in this workspace; the step wants it set and does not
+ * touch it: its plan is built through step.mid_q, which holds the counts of the
+ * plan's route chunks until the mid quantiser writes the mid rows there. */
 size_t q38m_moe_wide_workspace_bytes(uint32_t tokens);
 int q38m_moe_wide_workspace_bind(void* allocation, size_t bytes, uint32_t tokens,
                                  q38m_wide_workspace_v1* out);

@@ -706,10 +706,10 @@ int q38m_moe_prefill_wide_v1(const q38m_expert_weights_v1* gate_up,
     else
         status = q38m::launch_quantize_rows(hidden, tokens, Q38M_HIDDEN, ws->xq, ws->xs, s);
     if (status == hipSuccess)
-        // the chunk counts pass through the quantised mid rows, all of which
-        // the mid quantiser writes later: plan_scratch holds the counts of
-        // 2048-route chunks only (513 words per started 512 routes fit 128
-        // words per route from 5 routes on)
+        // the counts of the plan's chunks pass through the quantised mid rows,
+        // all of which the mid quantiser writes later (513 words per started
+        // 512 routes fit the rows' 128 words per route from 5 routes on);
+        // plan_scratch, sized for 2048-route chunks, would not hold them
         status = q38m::launch_step_wide_plan(ws->expert_ids, tokens, ws->plan,
                                              reinterpret_cast<uint32_t*>(ws->mid_q), s);
     if (status == hipSuccess)
