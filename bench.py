@@ -264,7 +264,7 @@ def pmc_report(workload, traffic_dir=None):
             "fetch": pmc_run("FETCH_SIZE", workload, f"--calibrate-copy-mib {mib}"),
             "write": pmc_run("WRITE_SIZE", workload, f"--calibrate-copy-mib {mib}")}
     lines = [f"# Kernel trace and hardware counters: `{workload}` workload", "",
-             f"Command (repository root on the GPU box): `python3 bench.py --pmc-report {workload}`.",
+             f"Command (repository root): `python3 bench.py --pmc-report {workload}`.",
              "It runs five child processes: `rocprofv3 --kernel-trace -f csv -d <tmp> -o pmc -- "
              f"python3 bench.py --no-counters {PMC_WORKLOADS[workload]}`, then the same with "
              "`--pmc <set>` for each counter set (FETCH/WRITE passes add "
@@ -864,7 +864,7 @@ def phase_report(tokens=8):
     rel = (rec["stamp"].astype(np.int64) - t0[:, None, None, None]) * 10 / 1000.0  # us
     layer_us = (rel[:, 1, :, len(DOWN_PHASES) - 1].max(axis=1))
     lines = ["# Batch-1 decode phases (config 3)", "",
-             "Command (repository root on the GPU box): `python3 bench.py --phase-report decode`.",
+             "Command (repository root): `python3 bench.py --phase-report decode`.",
              "", f"The timing build `libq38m_timed.so` (the product library with "
              "`-DQ38M_PHASE_TIMESTAMPS` in the decode kernels, `make timed`) runs "
              f"{tokens} tokens x {layers} layers of config 3 (W4 g32 gate/up, W8 per-channel "

@@ -1179,8 +1179,8 @@ bool launch_shared_tile(const uint16_t* hidden, const uint16_t* w_gate, const ui
 
 // Large products take workgroup tiles: 64 x 64 with three chunks in the ring
 // (three workgroups per CU) from about 200 tiles on, 128 x 128 with two (two
-// per CU) from about 400 of those.  Measured, old kernels / 64 x 64 / 128 x 128,
-// us -- router (512 x 2048): 1,024 rows 9.8 / 11.7 / 24.6, 2,048 rows 16.5 /
+// per CU) from about 400 of those.  Measured with row tiles dealt, old kernels /
+// 64 x 64 / 128 x 128, us -- router (512 x 2048): 1,024 rows 9.8 / 11.7 / 24.6, 2,048 rows 16.5 /
 // 12.6 / 24.4, 4,099 rows 31.2 / 19.7 / 25.6, 8,192 rows 54.0 / 31.1 / 28.6,
 // 32,768 rows 226 / 134 / 92.  Shared gate/up: 512 rows 11.1 / 14.9 / 33,
 // 1,024 rows 19.0 / 15.7 / 33, 4,099 rows 73.6 / 32.9 / 36.5, 32,768 rows
@@ -1301,8 +1301,12 @@ hipError_t launch_dense_gemm_act(const uint16_t* a, const uint16_t* b, uint32_t 
     return hipGetLastError();
 }
 
-// Above this many tokens the prepare's products run on workgroup tiles (a
-// prepare of up to 512 tokens leaves its stages in the scratch).
+// From this many tokens on the prepare's products run on workgroup tiles.  Not
+// the crossover: a prepare of up to 512 tokens leaves its stages (mix weights
+// among them) in the scratch, where tests/test_gpu_hyper.py compares them one by
+// one with the oracle.  Measured, us as stages / tiles, hidden 2,048 rank 320: 128
+// tokens 32.8 / 32.9, 320 38.1 / 35.7, 512 42.0 / 37.3; hidden 1,024 256 tokens
+// 26.0 / 27.2, 512 29.8 / 29.4; hidden 2,560 rank 96 128 tokens 37.3 / 33.8.
 constexpr uint32_t kHyperTileMinTokens = 513;
 
 bool launch_hyper_mix_down(const uint16_t* x, const uint16_t* mix_down, uint32_t tokens,

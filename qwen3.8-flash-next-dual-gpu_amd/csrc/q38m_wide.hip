@@ -298,18 +298,21 @@ __global__ __launch_bounds__(64) void wide_scatter_kernel(const int32_t* __restr
 // has its own L2; a task's slices next to each other on one XCD read the
 // same rows, and an expert's neighbouring tasks the same weights, from one
 // L2.  Two maps:
-// - up to kBlockedSlots task slots and in every wide_i8_kernel, XCD x gets the blocks of kTaskBlock
-//   consecutive tasks x, x + 8, x + 16, ...: the XCDs' loads are alike
-//   (contiguous eighths of the tasks differ by 10-30 % in rows for 1,500 to
-//   6,000 tokens), and the map needs no word of the plan, so a workgroup's
-//   first read is its task record; slots past the plan's tasks hold zero
-//   records.
+// - up to kBlockedSlots task slots, and in every wide_i8_kernel, XCD x gets the
+//   blocks of kTaskBlock consecutive tasks x, x + 8, x + 16, ...  The map needs
+//   no word of the plan, so a workgroup's first read is its task record;
+//   slots past the plan's tasks hold zero records.
 // - above, the kernels of groups of 32 and of W8 per-channel down give each
-//   XCD a contiguous eighth of the plan's tasks: the eighths are alike by
-//   then, and a hot expert's tasks stay in one L2.  32,768 tokens W4/W8, Zipf
-//   0.8: 3,073 us against 3,112 with blocks of four (16,384 tokens: 1,685
-//   against 1,678).  The 32x32 kernels keep the blocks (W4 groups of 128 at
-//   32,768 tokens 2.67 ms against 2.73 with eighths).
+//   XCD a contiguous eighth of the plan's tasks.
+// Contiguous eighths differ by 10-30 % in rows for 1,500 to 6,000 tokens, blocks
+// by less, but where the hot experts lie decides a single call: of eight
+// orders of popularity each gained or lost up to 10 %.  Means over them, step
+// in us as eighths / blocks, W4/W8: Zipf 0.8, 600 tokens 226 / 230, 1,500 348 / 338,
+// 2,500 465 / 448, 4,096 610 / 608, 8,192 982 / 958, 16,384 1,688 / 1,669; Zipf 1.1,
+// 1,500 273 / 269, 4,096 507 / 510, 8,192 872 / 864.  32,768 tokens (four orders):
+// uniform 3,024 / 3,087, Zipf 0.8 3,081 / 3,088, W4 in both 3,353 / 3,338: the
+// second map is kept for the first of these.  wide_i8_kernel at 32,768
+// tokens, W4 groups of 128, 2.73 / 2.67 ms.
 struct Placement {
     uint32_t task, slice;
 };
@@ -1015,11 +1018,14 @@ void down_w4g32_f16_kernel(const uint4* __restrict__ w, const uint16_t* __restri
 // the workgroup stages its int8 rows in a double-buffered 8 KB LDS image;
 // a wave's weights go straight to its registers, one to three steps ahead.
 //
-// What bounds it: the matrix cores and the VALU take turns on this part (a
-// microbenchmark of the two mixed at four VALU instructions per MFMA or more
-// takes the sum of their times), so a step costs its MFMAs plus its VALU
-// instructions.  The 32x32 form does twice the work of the 16x16x32 form
-// per matrix cycle and leaves a quarter of its cycles to the VALU.  The
+// What bounds it: the matrix cores and the VALU overlap only in part.  Three
+// waves per SIMD of independent v_mfma_i32_32x32x32_i8 and v_fma_f32 take, per
+// MFMA, 13.7 ns alone; with four v_fma_f32 (5.1 ns alone) 14.6, with eight (9.5)
+// 18.5, sixteen (19.4) 28.1, 32 (38.2) 45.4: from eight on about two thirds of the
+// MFMA's time come on top of the VALU's.  So both are kept few (here 17 to 22
+// VALU instructions per MFMA; 6,001 tokens in W4 groups of 128: MFMA busy 25 %,
+// VALU issue 50 %).  The 32x32 form does twice the work of the 16x16x32 form
+// per matrix cycle.  The
 // group chain is two VALU instructions per element: the MFMA accumulator
 // starts from the bits of 1.5 * 2^23, so its result read as a float is
 // 12582912 + acc exactly (|acc| < 2^22: 16 w a over 128 columns stays below
