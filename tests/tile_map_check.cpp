@@ -64,7 +64,7 @@ int main() {
                     }
                 }
                 for (uint32_t k : {320u, 2048u})
-                    for (uint64_t bytes : {uint64_t{0}, kXcdL2Bytes}) {
+                    for (uint64_t bytes : {uint64_t{0}, kInnerBytes}) {
                         const Shares& s = shares[tile_order(rows, columns, bytes, k)];
                         // (seven row tiles of few columns leave one XCD idle)
                         if (rows != 7u && static_cast<uint64_t>(rows) * columns >= 8u && s.least == 0u) {
