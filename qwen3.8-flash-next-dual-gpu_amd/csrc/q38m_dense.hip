@@ -1208,7 +1208,8 @@ constexpr uint64_t tile_count(uint32_t m, uint32_t n, uint32_t rows, uint32_t co
 //   2,048 10.2 / 11.4 / 23.4);
 // - whole K of three or four chunks, which hardly fill the ring, beside many
 //   columns (4,099 x 16,384 x 192 57.0 / 79.5 / 63.6; x 320 83.5 / 87.1 / 74.4;
-//   16,384 x 12,000 x 192 238 / - / 172), five to seven chunks of up to 64 rows
+//   16,384 x 12,000 x 192 238 / - / 172; 2,049 x 6,016 x 192 12.3 / - / 14.7, x 256
+//   14.0 / - / 14.1; 2,049 x 4,096 x 192 9.2 / - / 9.0), five to seven chunks of up to 64 rows
 //   (2 x 65,536 x 320 7.6 / 8.4 / -; x 512 10.6 / 10.6 / -).
 // 128 x 128 tiles need more than 64 rows and, over whole K, columns (64 x
 // 151,936 x 2,048 255 / 137 / 162; 131,072 x 64 x 320 16.1 / 16.4 / 20.4; K
@@ -1228,6 +1229,7 @@ bool launch_dense_large(const uint16_t* a, const uint16_t* b, uint32_t m, uint32
         if (m <= 32u || n <= 32u || (m <= 512u && tiles64 < 200u)) return false;
     } else {
         if (n >= 8192u && (m <= 64u ? k < 512u : k < 320u && m <= 8192u)) return false;
+        if (n >= 6000u && k < 256u && m <= 4608u) return false;
         tile128 = tile128 && n > 64u && !(k <= 512u && tiles128 > 512u && tiles128 <= 608u);
     }
     if (tile128)
