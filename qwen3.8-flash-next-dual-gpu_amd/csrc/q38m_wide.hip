@@ -1022,7 +1022,7 @@ void down_w4g32_f16_kernel(const uint4* __restrict__ w, const uint16_t* __restri
 // waves per SIMD of independent v_mfma_i32_32x32x32_i8 and v_fma_f32 take, per
 // MFMA, 13.7 ns alone; with four v_fma_f32 (5.1 ns alone) 14.6, with eight (9.5)
 // 18.5, sixteen (19.4) 28.1, 32 (38.2) 45.4: from eight on about two thirds of the
-// MFMA's time come on top of the VALU's.  So both are kept few (here 17 to 22
+// MFMA's time come on top of the VALU's.  So both are kept few (here 13 to 21
 // VALU instructions per MFMA; 6,001 tokens in W4 groups of 128: MFMA busy 25 %,
 // VALU issue 50 %).  The 32x32 form does twice the work of the 16x16x32 form
 // per matrix cycle.  The
