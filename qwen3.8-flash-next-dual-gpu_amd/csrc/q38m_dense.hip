@@ -1180,10 +1180,10 @@ bool launch_shared_tile(const uint16_t* hidden, const uint16_t* w_gate, const ui
 // Large products take workgroup tiles: 64 x 64 with three chunks in the ring
 // (three workgroups per CU) from about 200 tiles on, 128 x 128 with two (two
 // per CU) from about 400 of those.  Measured with row tiles dealt, old kernels /
-// 64 x 64 / 128 x 128, us -- router (512 x 2048): 1,024 rows 9.8 / 11.7 / 24.6, 2,048 rows 16.5 /
-// 12.6 / 24.4, 4,099 rows 31.2 / 19.7 / 25.6, 8,192 rows 54.0 / 31.1 / 28.6,
-// 32,768 rows 226 / 134 / 92.  Shared gate/up: 512 rows 11.1 / 14.9 / 33,
-// 1,024 rows 19.0 / 15.7 / 33, 4,099 rows 73.6 / 32.9 / 36.5, 32,768 rows
+// 64 x 64 / 128 x 128, us -- router (512 x 2048): 1,024 rows 9.8 / 11.7 / 24.6,
+// 2,048 rows 16.5 / 12.6 / 24.4, 4,099 rows 31.2 / 19.7 / 25.6, 8,192 rows 54.0 /
+// 31.1 / 28.6, 32,768 rows 226 / 134 / 92.  Shared gate/up: 512 rows 11.1 / 14.9 /
+// 33, 1,024 rows 19.0 / 15.7 / 33, 4,099 rows 73.6 / 32.9 / 36.5, 32,768 rows
 // 531 / 234 / 192.  Shared down (2,048 x 512): 512 rows 5.1 / 4.6 / -, 4,099
 // rows 20.5 / 16.9 / 17.9, 32,768 rows 125 / 136 / 101.
 constexpr uint32_t kTileMinTiles = 192;
@@ -1209,8 +1209,9 @@ constexpr uint64_t tile_count(uint32_t m, uint32_t n, uint32_t rows, uint32_t co
 // - whole K of three or four chunks, which hardly fill the ring, beside many
 //   columns (4,099 x 16,384 x 192 57.0 / 79.5 / 63.6; x 320 83.5 / 87.1 / 74.4;
 //   16,384 x 12,000 x 192 238 / - / 172; 2,049 x 6,016 x 192 12.3 / - / 14.7, x 256
-//   14.0 / - / 14.1; 2,049 x 4,096 x 192 9.2 / - / 9.0), five to seven chunks of up to 64 rows
-//   (2 x 65,536 x 320 7.6 / 8.4 / -; x 512 10.6 / 10.6 / -).
+//   14.0 / - / 14.1; 2,049 x 4,096 x 192 9.2 / 9.0 / 9.6), five to seven chunks of
+//   up to 64 rows (2 x 65,536 x 320 7.6 / 8.4 / -; 2 x 131,072 x 512 20.4 / 20.4 /
+//   22.9).
 // 128 x 128 tiles need more than 64 rows and, over whole K, columns (64 x
 // 151,936 x 2,048 255 / 137 / 162; 131,072 x 64 x 320 16.1 / 16.4 / 20.4; K
 // split, 65,536 x 64 x 2,048 72.9 / 47.0 / 43.8).  Two of them fit a CU: short
